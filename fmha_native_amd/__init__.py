@@ -172,7 +172,8 @@ def fmha_fwd_d64_bf16_ws(params, batch, causal, workspace=None, workspace_bytes=
                          variant=VARIANT_AUTO):
     """The launch with a workspace (device pointer as int, 256-byte aligned,
     at least :func:`workspace_size` bytes; None with 0 bytes allowed), which
-    lets dense causal launches with few heavy M-tiles run the balanced form.
+    lets dense causal launches with few heavy M-tiles run the balanced form and
+    launches of few query rows split their keys over blocks.
     ``variant``: VARIANT_AUTO, VARIANT_BALANCED, VARIANT_BALANCED_PAIR or any
     other (workspace unused).  Raises :class:`FmhaError` on a non-zero hipError_t."""
     rc = load_library().fmha_fwd_d64_bf16_ws(ctypes.byref(params), int(batch), int(causal), int(variant), workspace,
@@ -220,8 +221,10 @@ def check_params(params, batch, causal):
 
 
 def pick_variant(params, batch, causal, compute_units=0):
-    """The form VARIANT_AUTO resolves to on a device with ``compute_units``
-    CUs (0 = the current device's); -1 for rejected arguments.  Host only."""
+    """The M-tile form VARIANT_AUTO resolves to on a device with
+    ``compute_units`` CUs (0 = the current device's), where the decode form
+    (few query rows, no code of its own) does not take the launch; -1 for
+    rejected arguments.  Host only."""
     return load_library().fmha_fwd_d64_bf16_pick_variant(ctypes.byref(params), int(batch), int(causal),
                                                           int(compute_units))
 

@@ -72,6 +72,7 @@ def build(verbose=False):
         objs = {
             "kernel": os.path.join(tmp, "fmha_fwd_kernel.o"),
             "api": os.path.join(tmp, "fmha_fwd_api.o"),
+            "decode": os.path.join(tmp, "fmha_decode.o"),
             "merge": os.path.join(tmp, "fmha_merge.o"),
             "noalloc": os.path.join(tmp, "fmha_noalloc.o"),
             "runner": os.path.join(tmp, "runner.o"),
@@ -79,6 +80,7 @@ def build(verbose=False):
         _run_all([
             [HIPCC, *HIP_FLAGS, "-c", os.path.join(CSRC, "fmha_fwd_kernel.hip"), "-o", objs["kernel"]],
             [HIPCC, *HIP_FLAGS, "-c", os.path.join(CSRC, "fmha_fwd_api.hip"), "-o", objs["api"]],
+            [HIPCC, *HIP_FLAGS, "-c", os.path.join(CSRC, "fmha_decode.hip"), "-o", objs["decode"]],
             [HIPCC, *HIP_FLAGS, "-c", os.path.join(CSRC, "fmha_merge.hip"), "-o", objs["merge"]],
             [HIPCC, *HIP_FLAGS, "-c", os.path.join(CSRC, "fmha_noalloc.hip"), "-o", objs["noalloc"]],
             ["g++", "-O3", "-fopenmp", "-fPIC", "-std=c++17", f"-I{CSRC}", "-c",
@@ -88,7 +90,7 @@ def build(verbose=False):
         ], verbose)
         os.replace(ORACLE_LIB + ".tmp", ORACLE_LIB)
         tmp_lib = os.path.join(tmp, "libfmha_native_amd.so")
-        _run_all([[HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", objs["kernel"], objs["api"], objs["merge"], objs["noalloc"], objs["runner"],
+        _run_all([[HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", objs["kernel"], objs["api"], objs["decode"], objs["merge"], objs["noalloc"], objs["runner"],
                    "-lgomp", "-o", tmp_lib]], verbose)
         shutil.copyfile(tmp_lib, LIB + ".tmp")
         os.replace(LIB + ".tmp", LIB)

@@ -236,6 +236,88 @@ int pick_form(const FmhaFwdParams* p, int batch, int causal, int64_t cus) {
     return pick_variant(grid_blocks(p, batch), pair_blocks(p, batch), causal, p->seqlen_k, cus);
 }
 
+// ---- decode form (fmha_decode.hip) ----
+// The packed rows of a KV head: its query heads x the queries.
+int64_t decode_rows(const FmhaFwdParams* p) { return (int64_t)(p->nhead_q / p->nhead_k) * p->seqlen_q; }
+// Whether a launch runs it: the automatic choice without an order flag (those
+// ask for the M-tile grid); the bounds steer varlen launches.
+// Against the M-tile forms on one box (dense caches, LSE, us before / after):
+// B16 H32/8 1 x 4100 82 / 28, B1 H32/8 1 x 32768 312 / 18, B2 H16/2 16 x 16384
+// 77 / 13, B64 H16/16 1 x 128 11.5 / 10.8, B16 H16/16 64 x 4096 62 / 53; past
+// 32 queries short key ranges lose (64 x 200 17 / 22) and past 64 the M-tile
+// forms win (128 x 4096 64 / 87: four row tiles re-read K and V).
+bool takes_decode(const FmhaFwdParams* p, int variant) {
+    return variant == FMHA_VARIANT_AUTO && p->seqlen_q > 0 && decode_rows(p) <= FMHA_DECODE_MAX_ROWS &&
+           p->seqlen_k >= 128 && (p->seqlen_q <= 32 || (p->seqlen_q <= 64 && p->seqlen_k >= 1024));
+}
+// Fills `a` but its workspace pointers for at most `chunks` key chunks per
+// (sequence, KV head), whole steps each; returns the workspace bytes.
+int64_t decode_plan(const FmhaFwdParams* p, int batch, int chunks, int64_t cus, FmhaDecodeArgs* a) {
+    const int steps = std::max(1, (p->seqlen_k + FMHA_DECODE_KEY_STEP - 1) / FMHA_DECODE_KEY_STEP);
+    const int per = (steps + chunks - 1) / chunks;
+    a->p = *p;
+    a->part = a->ml = nullptr;
+    a->chunk_keys = per * FMHA_DECODE_KEY_STEP;
+    a->n_chunks = (steps + per - 1) / per;
+    a->rows = (int)decode_rows(p);
+    const int64_t pairs = (int64_t)batch * p->nhead_k;
+    const int64_t blocks = pairs * a->n_chunks * ((a->rows + FMHA_DECODE_ROWS - 1) / FMHA_DECODE_ROWS);
+    // eight waves (one block per CU) halve a block's serial chain; short key
+    // ranges on more blocks than CUs take two four-wave blocks per CU, whose
+    // prologues and epilogues overlap (B64 H16/16 1 x 128: 14.9 / 10.8 us with
+    // 8 / 4 waves; 1 x 2048 on 320 blocks 36.2 / 34.7; 1 x 8000 varlen on 320
+    // 80.6 / 96.6)
+    a->waves = blocks > cus && p->seqlen_k <= 2048 ? 4 : 8;
+    return a->n_chunks == 1 ? 0 : pairs * a->n_chunks * a->rows * (FMHA_HEAD_DIM + 2) * (int64_t)sizeof(float);
+}
+// Key chunks of a launch with a workspace: none where the pairs fill half the
+// CUs (B16 H32/8 1 x 4100, 128 blocks: 28.7 us whole, 29.2 in two chunks; B64
+// H8/2 1 x 2048 13.4 / 16.2) or the chain is at most five steps (the merge
+// launch costs ~3 us, a step 0.6: B1 H8 4 x 4096, 16 steps, 15.7 whole, 9.8 in
+// eight chunks); else as many as fit the CUs in one round (12 sequences to
+// 16,000 keys, 24 pairs: 10 chunks 16.3 us, 16 chunks, a partial second round,
+// 19.7).
+int decode_chunks(const FmhaFwdParams* p, int batch, int64_t cus) {
+    const int64_t items =
+        (int64_t)batch * p->nhead_k * ((decode_rows(p) + FMHA_DECODE_ROWS - 1) / FMHA_DECODE_ROWS);
+    if (items <= 0 || 2 * items >= cus || p->seqlen_k <= 5 * FMHA_DECODE_KEY_STEP) return 1;
+    return (int)std::min<int64_t>(FMHA_DECODE_MAX_CHUNKS, cus / items);
+}
+hipError_t decode_launch(const FmhaDecodeArgs& a, int batch, int causal, hipStream_t stream) {
+    using Entry = void (*)(FmhaDecodeArgs);
+    static const Entry walk[2][2][2] = {
+        {{fmha_fwd_d64_bf16_decode_msk0, fmha_fwd_d64_bf16_decode_msk0_varlen},
+         {fmha_fwd_d64_bf16_decode_msk1, fmha_fwd_d64_bf16_decode_msk1_varlen}},
+        {{fmha_fwd_d64_bf16_decode4_msk0, fmha_fwd_d64_bf16_decode4_msk0_varlen},
+         {fmha_fwd_d64_bf16_decode4_msk1, fmha_fwd_d64_bf16_decode4_msk1_varlen}}};
+    static const Entry merge[2][2] = {
+        {fmha_fwd_d64_bf16_decode_merge_msk0, fmha_fwd_d64_bf16_decode_merge_msk0_varlen},
+        {fmha_fwd_d64_bf16_decode_merge_msk1, fmha_fwd_d64_bf16_decode_merge_msk1_varlen}};
+    const int c = causal ? 1 : 0, v = a.p.seqstart_q != nullptr ? 1 : 0;
+    hipLaunchKernelGGL(walk[a.waves == 4 ? 1 : 0][c][v],
+                       dim3(a.p.nhead_k * a.n_chunks, (a.rows + FMHA_DECODE_ROWS - 1) / FMHA_DECODE_ROWS, batch),
+                       dim3(64 * a.waves), 0, stream, a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || a.n_chunks == 1) return e;
+    hipLaunchKernelGGL(merge[c][v],
+                       dim3((a.rows + FMHA_DECODE_MERGE_ROWS - 1) / FMHA_DECODE_MERGE_ROWS, a.p.nhead_k, batch),
+                       dim3(64 * FMHA_DECODE_MERGE_ROWS), 0, stream, a);
+    return hipGetLastError();
+}
+// The launch with as many chunks as the workspace holds: the plan's, or one.
+hipError_t decode_run(const FmhaFwdParams* p, int batch, int causal, void* workspace, int64_t workspace_bytes,
+                      hipStream_t stream) {
+    FmhaDecodeArgs a;
+    const int64_t cus = device_cus();
+    if (decode_plan(p, batch, decode_chunks(p, batch, cus), cus, &a) > workspace_bytes)
+        decode_plan(p, batch, 1, cus, &a);
+    if (a.n_chunks > 1) {
+        a.part = (float*)workspace;
+        a.ml = a.part + (int64_t)batch * p->nhead_k * a.n_chunks * a.rows * FMHA_HEAD_DIM;
+    }
+    return decode_launch(a, batch, causal, stream);
+}
+
 }  // namespace
 
 namespace {
@@ -453,16 +535,25 @@ extern "C" int fmha_fwd_d64_bf16_balanced_plan(const FmhaFwdParams* p, int batch
     return a.n_items;
 }
 
-extern "C" int64_t fmha_fwd_d64_bf16_workspace_size(const FmhaFwdParams* p, int batch, int causal, int variant) {
+int64_t fmha_balanced_workspace_size(const FmhaFwdParams* p, int batch, int causal, int variant) {
     if (fmha_fwd_d64_bf16_check(p, batch, causal) != hipSuccess) return -1;
     if (order_of(variant) < 0) return -1;
     const int mode = plan_mode(variant & ~kOrderFlags);
     if (mode < 0) return 0;
+    if (takes_decode(p, variant)) return 0;
     int64_t bytes = 0;
     // the same plan (and cache entry) as the launch with this variant
     const int xccs = order_of(variant) == kOrderReference ? 1 : device_shape().xccs;
     if (!balanced_plan(p, batch, causal, device_cus(), xccs, mode, nullptr, &bytes)) return 0;
     return bytes;
+}
+
+extern "C" int64_t fmha_fwd_d64_bf16_workspace_size(const FmhaFwdParams* p, int batch, int causal, int variant) {
+    const int64_t bytes = fmha_balanced_workspace_size(p, batch, causal, variant);
+    if (bytes != 0 || !takes_decode(p, variant)) return bytes;
+    FmhaDecodeArgs a;
+    const int64_t cus = device_cus();
+    return decode_plan(p, batch, decode_chunks(p, batch, cus), cus, &a);
 }
 
 extern "C" hipError_t fmha_fwd_d64_bf16_ws(const FmhaFwdParams* p, int batch, int causal, int variant,
@@ -476,6 +567,7 @@ extern "C" hipError_t fmha_fwd_d64_bf16_ws(const FmhaFwdParams* p, int batch, in
         (reinterpret_cast<uintptr_t>(workspace) & 255u))
         return hipErrorInvalidValue;
     if (batch == 0 || p->seqlen_q == 0) return hipSuccess;
+    if (takes_decode(p, variant)) return decode_run(p, batch, causal, workspace, workspace_bytes, stream);
     FmhaBalancedArgs a;
     int64_t need = 0;
     // the reference-order flag keeps the plain heaviest-first table (the
@@ -508,6 +600,7 @@ extern "C" int fmha_fwd_d64_bf16_pick_variant(const FmhaFwdParams* p, int batch,
 extern "C" int fmha_fwd_d64_bf16_tile_major(const FmhaFwdParams* p, int batch, int causal) {
     if (fmha_fwd_d64_bf16_check(p, batch, causal) != hipSuccess) return -1;
     if (p->seqlen_q == 0 || batch == 0) return 0;  // nothing is launched
+    if (takes_decode(p, FMHA_VARIANT_AUTO)) return 0;
     if (dense_tile_major(p, batch, causal, kOrderAuto)) return 1;
     // varlen: the compact orders, which only the regular form has
     if (pick_form(p, batch, causal, device_cus()) != FMHA_VARIANT_REGULAR) return 0;
@@ -522,6 +615,7 @@ extern "C" hipError_t fmha_fwd_d64_bf16_variant(const FmhaFwdParams* p, int batc
     const int order = order_of(variant);
     if (order < 0) return hipErrorInvalidValue;  // more than one order flag
     const bool tile_major = dense_tile_major(p, batch, causal, order);
+    const bool decode = takes_decode(p, variant);
     variant &= ~kOrderFlags;
     // the balanced forms need fmha_fwd_d64_bf16_ws; 4 is a retired value
     if (!(variant == FMHA_VARIANT_AUTO || variant == FMHA_VARIANT_REGULAR || variant == FMHA_VARIANT_SPLITKV ||
@@ -530,6 +624,7 @@ extern "C" hipError_t fmha_fwd_d64_bf16_variant(const FmhaFwdParams* p, int batc
     const bool varlen = p->seqstart_q != nullptr;
     if (variant == FMHA_VARIANT_PAIR_STREAM && varlen) return hipErrorInvalidValue;  // dense layouts only
     if (batch == 0 || p->seqlen_q == 0) return hipSuccess;  // nothing to compute
+    if (decode) return decode_run(p, batch, causal, nullptr, 0, stream);
     const int m_tiles = (p->seqlen_q + kM0 - 1) / kM0;
     const dim3 grid(p->nhead_q, m_tiles, batch);
     if (variant == FMHA_VARIANT_PAIR_STREAM) {

@@ -33,3 +33,37 @@ struct FmhaStreamArgs {
 };
 __global__ void fmha_fwd_d64_bf16_pair_stream_msk0(FmhaStreamArgs args);
 __global__ void fmha_fwd_d64_bf16_pair_stream_msk1(FmhaStreamArgs args);
+
+// Decode form (see fmha_decode.hip): packed query rows of one KV head over
+// key chunks.
+#define FMHA_DECODE_ROWS 32                            // packed rows (query heads of a KV head x tokens) per block
+#define FMHA_DECODE_KEY_STEP 256                       // keys eight waves take per step; chunks are multiples of it
+#define FMHA_DECODE_MAX_ROWS 128                       // packed rows per KV head a launch may have
+#define FMHA_DECODE_MAX_CHUNKS 64                      // the merge holds one chunk's weight per lane
+#define FMHA_DECODE_MERGE_ROWS 4                       // rows (waves) per merge block
+struct FmhaDecodeArgs {
+    FmhaFwdParams p;
+    float* part;     // [batch][nhead_k][n_chunks][rows][64] unnormalised O (n_chunks > 1)
+    float* ml;       // [batch][nhead_k][n_chunks][rows][2] row max (scaled) and row sum
+    int n_chunks;    // key chunks per (sequence, KV head)
+    int chunk_keys;  // keys per chunk (the last takes the rest)
+    int waves;       // waves per block: 8 (decode entries) or 4 (decode4)
+    int rows;        // packed rows per (sequence, KV head): nhead_q / nhead_k * seqlen_q
+};
+__global__ void fmha_fwd_d64_bf16_decode_msk0(FmhaDecodeArgs args);
+__global__ void fmha_fwd_d64_bf16_decode_msk1(FmhaDecodeArgs args);
+__global__ void fmha_fwd_d64_bf16_decode_msk0_varlen(FmhaDecodeArgs args);
+__global__ void fmha_fwd_d64_bf16_decode_msk1_varlen(FmhaDecodeArgs args);
+__global__ void fmha_fwd_d64_bf16_decode4_msk0(FmhaDecodeArgs args);
+__global__ void fmha_fwd_d64_bf16_decode4_msk1(FmhaDecodeArgs args);
+__global__ void fmha_fwd_d64_bf16_decode4_msk0_varlen(FmhaDecodeArgs args);
+__global__ void fmha_fwd_d64_bf16_decode4_msk1_varlen(FmhaDecodeArgs args);
+__global__ void fmha_fwd_d64_bf16_decode_merge_msk0(FmhaDecodeArgs args);
+__global__ void fmha_fwd_d64_bf16_decode_merge_msk1(FmhaDecodeArgs args);
+__global__ void fmha_fwd_d64_bf16_decode_merge_msk0_varlen(FmhaDecodeArgs args);
+__global__ void fmha_fwd_d64_bf16_decode_merge_msk1_varlen(FmhaDecodeArgs args);
+
+// fmha_fwd_d64_bf16_workspace_size for the balanced forms alone (the entry
+// point on the static array splits no decode launch: calls on several streams
+// that needed no scratch must not start to share it).
+int64_t fmha_balanced_workspace_size(const FmhaFwdParams* p, int batch, int causal, int variant);

@@ -16,6 +16,7 @@
 #include <atomic>
 
 #include "fmha_fwd.h"
+#include "fmha_internal.h"
 
 static __device__ __align__(256) char scratch[FMHA_NOALLOC_SCRATCH_BYTES];
 
@@ -46,7 +47,7 @@ hipError_t scratch_here(void** out) {
 
 extern "C" hipError_t fmha_fwd_d64_bf16_noalloc(const FmhaFwdParams* params, int batch, int causal, int variant,
                                                 hipStream_t stream) {
-    const int64_t need = fmha_fwd_d64_bf16_workspace_size(params, batch, causal, variant);
+    const int64_t need = fmha_balanced_workspace_size(params, batch, causal, variant);
     if (need < 0) return hipErrorInvalidValue;                                  // rejected arguments
     if (need > (int64_t)FMHA_NOALLOC_SCRATCH_BYTES) return hipErrorInvalidValue;  // beyond the array
     void* ptr = nullptr;

@@ -114,7 +114,10 @@ hipError_t fmha_fwd_d64_bf16(const FmhaFwdParams* params, int batch, int causal,
 
 /* The same launch with the kernel form chosen by the caller (this build's
  * own; no counterpart in the reference):
- *   FMHA_VARIANT_AUTO     what fmha_fwd_d64_bf16() picks: short for
+ *   FMHA_VARIANT_AUTO     what fmha_fwd_d64_bf16() picks: the decode form (below)
+ *                         for at most 32 queries (64 from 1024 keys on), at
+ *                         most 128 rows per KV head (nhead_q / nhead_k x
+ *                         seqlen_q), seqlen_k >= 128 and no order flag; short for
  *                         launches with seqlen_k <= 192 and at least
  *                         2 x CUs x 128 query rows (batch x nhead_q x
  *                         seqlen_q; varlen: the bounds), or causal with
@@ -143,6 +146,11 @@ hipError_t fmha_fwd_d64_bf16(const FmhaFwdParams* params, int batch, int causal,
  *                         taking every CU-count-th pair; causal: one block
  *                         per pair of the first half of each (batch, head),
  *                         taking that pair's mirror next
+ * The decode form has no code of its own: the query heads of a KV head share
+ * one pass over its keys, whose 32-key steps the waves of a block split, and
+ * with a workspace (fmha_fwd_d64_bf16_ws) the blocks too.  In varlen launches
+ * seqlen_q must bound every sequence's queries (rows past it are not
+ * computed); seqlen_k only steers the choice and the split.
  * All forms give the same results up to fp32 rounding order.  Causal dense
  * launches of more than one batch whose K/V per XCD, batch x ceil(nhead_k/8)
  * x seqlen_k x 256 bytes, is at most 8 MiB run the form's tile-major entry
@@ -190,7 +198,11 @@ hipError_t fmha_fwd_d64_bf16_variant(const FmhaFwdParams* params, int batch, int
  * (fp32, the same merge as the split-KV form; results equal the other forms
  * up to fp32 rounding order).
  *   variant: FMHA_VARIANT_AUTO (balanced when it applies and the workspace
- *            is large enough, else what fmha_fwd_d64_bf16 picks),
+ *            is large enough; the decode form, its keys split over
+ *            blocks where the (sequence, KV head) pairs fill less than half
+ *            the compute units and seqlen_k > 1280: each block's fp32 partial
+ *            goes to the workspace and a second launch merges them, unsplit
+ *            if the workspace is too small; else what fmha_fwd_d64_bf16 picks),
  *            FMHA_VARIANT_BALANCED (always the balanced form, with the
  *            heavy-M-tile rule applied even where the regular order would
  *            balance: causal dense only; hipErrorInvalidValue if it cannot
@@ -224,6 +236,7 @@ int64_t fmha_fwd_d64_bf16_workspace_size(const FmhaFwdParams* params, int batch,
  * until the process ends; a launch whose plan needs more returns
  * hipErrorInvalidValue and launches nothing (the balanced form needs
  * 2 x 34,816 bytes per split M-tile: B1 H2 S40000 causal needs 30,359,552).
+ * The decode form runs unsplit here: it uses none of the array.
  * Calls that overlap in time on one GPU share the array and race; calls in
  * stream order do not (nothing in it needs clearing).  Allocates nothing. */
 #define FMHA_NOALLOC_SCRATCH_BYTES (32 << 20)
@@ -250,7 +263,8 @@ int fmha_fwd_d64_bf16_balanced_plan(const FmhaFwdParams* params, int batch, int 
  * needed).  Returns hipSuccess or hipErrorInvalidValue. */
 hipError_t fmha_fwd_d64_bf16_check(const FmhaFwdParams* params, int batch, int causal);
 
-/* The form FMHA_VARIANT_AUTO resolves to for these arguments on a device with
+/* The M-tile form FMHA_VARIANT_AUTO resolves to where the decode form does not
+ * take the launch, for these arguments on a device with
  * `compute_units` compute units (0 = the current device's count), without
  * launching (this build's own; no counterpart in the reference).  Returns
  * FMHA_VARIANT_REGULAR, _SPLITKV, _PAIR or _SHORT, or -1 for rejected
