@@ -236,88 +236,6 @@ int pick_form(const FmhaFwdParams* p, int batch, int causal, int64_t cus) {
     return pick_variant(grid_blocks(p, batch), pair_blocks(p, batch), causal, p->seqlen_k, cus);
 }
 
-// ---- decode form (fmha_decode.hip) ----
-// The packed rows of a KV head: its query heads x the queries.
-int64_t decode_rows(const FmhaFwdParams* p) { return (int64_t)(p->nhead_q / p->nhead_k) * p->seqlen_q; }
-// Whether a launch runs it: the automatic choice without an order flag (those
-// ask for the M-tile grid); the bounds steer varlen launches.
-// Against the M-tile forms on one box (dense caches, LSE, us before / after):
-// B16 H32/8 1 x 4100 82 / 28, B1 H32/8 1 x 32768 312 / 18, B2 H16/2 16 x 16384
-// 77 / 13, B64 H16/16 1 x 128 11.5 / 10.8, B16 H16/16 64 x 4096 62 / 53; past
-// 32 queries short key ranges lose (64 x 200 17 / 22) and past 64 the M-tile
-// forms win (128 x 4096 64 / 87: four row tiles re-read K and V).
-bool takes_decode(const FmhaFwdParams* p, int variant) {
-    return variant == FMHA_VARIANT_AUTO && p->seqlen_q > 0 && decode_rows(p) <= FMHA_DECODE_MAX_ROWS &&
-           p->seqlen_k >= 128 && (p->seqlen_q <= 32 || (p->seqlen_q <= 64 && p->seqlen_k >= 1024));
-}
-// Fills `a` but its workspace pointers for at most `chunks` key chunks per
-// (sequence, KV head), whole steps each; returns the workspace bytes.
-int64_t decode_plan(const FmhaFwdParams* p, int batch, int chunks, int64_t cus, FmhaDecodeArgs* a) {
-    const int steps = std::max(1, (p->seqlen_k + FMHA_DECODE_KEY_STEP - 1) / FMHA_DECODE_KEY_STEP);
-    const int per = (steps + chunks - 1) / chunks;
-    a->p = *p;
-    a->part = a->ml = nullptr;
-    a->chunk_keys = per * FMHA_DECODE_KEY_STEP;
-    a->n_chunks = (steps + per - 1) / per;
-    a->rows = (int)decode_rows(p);
-    const int64_t pairs = (int64_t)batch * p->nhead_k;
-    const int64_t blocks = pairs * a->n_chunks * ((a->rows + FMHA_DECODE_ROWS - 1) / FMHA_DECODE_ROWS);
-    // eight waves (one block per CU) halve a block's serial chain; short key
-    // ranges on more blocks than CUs take two four-wave blocks per CU, whose
-    // prologues and epilogues overlap (B64 H16/16 1 x 128: 14.9 / 10.8 us with
-    // 8 / 4 waves; 1 x 2048 on 320 blocks 36.2 / 34.7; 1 x 8000 varlen on 320
-    // 80.6 / 96.6)
-    a->waves = blocks > cus && p->seqlen_k <= 2048 ? 4 : 8;
-    return a->n_chunks == 1 ? 0 : pairs * a->n_chunks * a->rows * (FMHA_HEAD_DIM + 2) * (int64_t)sizeof(float);
-}
-// Key chunks of a launch with a workspace: none where the pairs fill half the
-// CUs (B16 H32/8 1 x 4100, 128 blocks: 28.7 us whole, 29.2 in two chunks; B64
-// H8/2 1 x 2048 13.4 / 16.2) or the chain is at most five steps (the merge
-// launch costs ~3 us, a step 0.6: B1 H8 4 x 4096, 16 steps, 15.7 whole, 9.8 in
-// eight chunks); else as many as fit the CUs in one round (12 sequences to
-// 16,000 keys, 24 pairs: 10 chunks 16.3 us, 16 chunks, a partial second round,
-// 19.7).
-int decode_chunks(const FmhaFwdParams* p, int batch, int64_t cus) {
-    const int64_t items =
-        (int64_t)batch * p->nhead_k * ((decode_rows(p) + FMHA_DECODE_ROWS - 1) / FMHA_DECODE_ROWS);
-    if (items <= 0 || 2 * items >= cus || p->seqlen_k <= 5 * FMHA_DECODE_KEY_STEP) return 1;
-    return (int)std::min<int64_t>(FMHA_DECODE_MAX_CHUNKS, cus / items);
-}
-hipError_t decode_launch(const FmhaDecodeArgs& a, int batch, int causal, hipStream_t stream) {
-    using Entry = void (*)(FmhaDecodeArgs);
-    static const Entry walk[2][2][2] = {
-        {{fmha_fwd_d64_bf16_decode_msk0, fmha_fwd_d64_bf16_decode_msk0_varlen},
-         {fmha_fwd_d64_bf16_decode_msk1, fmha_fwd_d64_bf16_decode_msk1_varlen}},
-        {{fmha_fwd_d64_bf16_decode4_msk0, fmha_fwd_d64_bf16_decode4_msk0_varlen},
-         {fmha_fwd_d64_bf16_decode4_msk1, fmha_fwd_d64_bf16_decode4_msk1_varlen}}};
-    static const Entry merge[2][2] = {
-        {fmha_fwd_d64_bf16_decode_merge_msk0, fmha_fwd_d64_bf16_decode_merge_msk0_varlen},
-        {fmha_fwd_d64_bf16_decode_merge_msk1, fmha_fwd_d64_bf16_decode_merge_msk1_varlen}};
-    const int c = causal ? 1 : 0, v = a.p.seqstart_q != nullptr ? 1 : 0;
-    hipLaunchKernelGGL(walk[a.waves == 4 ? 1 : 0][c][v],
-                       dim3(a.p.nhead_k * a.n_chunks, (a.rows + FMHA_DECODE_ROWS - 1) / FMHA_DECODE_ROWS, batch),
-                       dim3(64 * a.waves), 0, stream, a);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess || a.n_chunks == 1) return e;
-    hipLaunchKernelGGL(merge[c][v],
-                       dim3((a.rows + FMHA_DECODE_MERGE_ROWS - 1) / FMHA_DECODE_MERGE_ROWS, a.p.nhead_k, batch),
-                       dim3(64 * FMHA_DECODE_MERGE_ROWS), 0, stream, a);
-    return hipGetLastError();
-}
-// The launch with as many chunks as the workspace holds: the plan's, or one.
-hipError_t decode_run(const FmhaFwdParams* p, int batch, int causal, void* workspace, int64_t workspace_bytes,
-                      hipStream_t stream) {
-    FmhaDecodeArgs a;
-    const int64_t cus = device_cus();
-    if (decode_plan(p, batch, decode_chunks(p, batch, cus), cus, &a) > workspace_bytes)
-        decode_plan(p, batch, 1, cus, &a);
-    if (a.n_chunks > 1) {
-        a.part = (float*)workspace;
-        a.ml = a.part + (int64_t)batch * p->nhead_k * a.n_chunks * a.rows * FMHA_HEAD_DIM;
-    }
-    return decode_launch(a, batch, causal, stream);
-}
-
 }  // namespace
 
 namespace {
@@ -510,6 +428,290 @@ bool balanced_plan_build(const FmhaFwdParams* p, int batch, int causal, int64_t 
     return true;
 }
 
+// ---- chunk form (kModeChunk in fmha_fwd_kernel.hip) ----
+//
+// Dense launches of at most 0.6 M-tiles per compute unit, with a workspace.
+// What bounds them is one block's chain of key tiles (split-KV halves it,
+// the balanced form too), so M-tiles of more than `tiles` key tiles are cut
+// into equal chunks that run as blocks of their own, all resident at once, and
+// a second launch merges the partial results.  Measured on 256 CUs over 29
+// shapes (16-144 M-tiles of 11-313 key tiles, 12 chunk lengths each), a launch
+// of I chunk blocks, the longest of w tiles, at most c per M-tile, takes
+//     6.1 + k (w + 1) + 0.0127 I + 0.3 c   us,
+// k = 0.55 up to one block per CU and 0.9 up to two (rms error 8 %): shorter
+// chunks trade the chain against the partials' traffic and the merge's.  The
+// forms without chunks take 9.5 + 0.275 n us (balanced), 6 + 0.435 n
+// (split-KV) or 3.9 + 0.55 n (regular) for their longest M-tile's n tiles.
+// The rule takes the chunk length with the least estimate where that is below
+// the other form's.  Start / chunks: B1 H16 512 x 16384 causal 78 / 46 us,
+// H16 100 x 8192 43 / 18, H2 S4096 causal 26 / 17, H1 S16384 causal 80 / 53,
+// H4 S4096 34 / 29, H6 S2500 23.7 / 21.5; H16 S1024 (128 M-tiles of 16 tiles)
+// stays regular, 12.5 / 14.
+struct ChunkChoice {
+    int tiles;  // key tiles per chunk
+    double us;  // estimate
+};
+int chunk_count(int n, int tiles) { return std::max(1, (n + tiles - 1) / tiles); }
+// Key tiles of M-tile mt.
+int mtile_tiles(const FmhaFwdParams* p, int causal, int mt) {
+    return causal ? causal_ntiles(p, mt) : (p->seqlen_k + kN0 - 1) / kN0;
+}
+// Chunk blocks of a launch (M-tiles kept whole among them).
+int64_t chunk_items(const FmhaFwdParams* p, int causal, int m_tiles, int64_t hb, int tiles) {
+    if (!causal) return hb * m_tiles * chunk_count(mtile_tiles(p, 0, 0), tiles);
+    int64_t n = 0;
+    for (int mt = 0; mt < m_tiles; ++mt) n += chunk_count(causal_ntiles(p, mt), tiles);
+    return hb * n;
+}
+// The chunk length for at most `slots` blocks at k us per tile.
+ChunkChoice chunk_choice(const FmhaFwdParams* p, int causal, int m_tiles, int64_t hb, int longest, double total,
+                         int64_t slots, double k) {
+    // the estimate's minimum over the length, then as long as the blocks fit
+    int lo = std::max(4, (int)std::sqrt((0.0127 * total + 0.3 * longest) / k));
+    int hi = longest;  // every M-tile whole: fewer blocks than CUs (the caller's condition)
+    if (lo < hi && chunk_items(p, causal, m_tiles, hb, lo) > slots) {
+        while (hi - lo > 1) {  // items(lo) > slots >= items(hi)
+            const int mid = (lo + hi) / 2;
+            (chunk_items(p, causal, m_tiles, hb, mid) > slots ? lo : hi) = mid;
+        }
+        lo = hi;
+    }
+    if (lo >= longest) return {0, 0.0};
+    const int c = std::min(FMHA_CHUNK_MAX_CHUNKS, chunk_count(longest, lo));
+    const double w = (longest + c - 1) / c;
+    return {lo, 6.1 + k * (w + 1.0) + 0.0127 * (double)chunk_items(p, causal, m_tiles, hb, lo) + 0.3 * c};
+}
+// The M-tile forms' estimate for launches of at most one block per CU, and
+// the chunk length (0: no chunks).
+ChunkChoice mtile_us(const FmhaFwdParams* p, int batch, int causal, int64_t cus, bool workspace) {
+    const int m_tiles = (p->seqlen_q + kM0 - 1) / kM0;
+    const int64_t hb = (int64_t)p->nhead_q * batch;
+    const int longest = mtile_tiles(p, causal, m_tiles - 1);
+    ChunkChoice best{0, p->seqlen_k >= 2048 ? 6.0 + 0.435 * longest : std::max(6.7, 3.9 + 0.55 * longest)};
+    if (!workspace || p->seqstart_q != nullptr || hb > cus || hb * m_tiles > cus) return best;
+    double total = 0.0;
+    for (int mt = 0; mt < m_tiles; ++mt) total += mtile_tiles(p, causal, mt);
+    total *= (double)hb;
+    if (causal && balanced_pays(hb * m_tiles, longest, total / (2.0 * (double)cus), cus))
+        best.us = 9.5 + 0.275 * longest;
+    if (8 * hb * m_tiles > 5 * cus || m_tiles > FMHA_CHUNK_MAX_MTILES) return best;  // chunks: the measured range
+    for (const ChunkChoice& c : {chunk_choice(p, causal, m_tiles, hb, longest, total, cus, 0.55),
+                                 chunk_choice(p, causal, m_tiles, hb, longest, total, 2 * cus, 0.9)})
+        if (c.tiles > 0 && c.us < (best.tiles == 0 ? 0.97 : 1.0) * best.us) best = c;
+    return best;
+}
+
+// ---- decode form (fmha_decode.hip) ----
+// The packed rows of a KV head (its query heads x the queries) and the blocks
+// of an unsplit launch.
+int64_t decode_rows(const FmhaFwdParams* p) { return (int64_t)(p->nhead_q / p->nhead_k) * p->seqlen_q; }
+int64_t decode_items(const FmhaFwdParams* p, int batch) {
+    const int64_t tiles = (decode_rows(p) + FMHA_DECODE_ROWS - 1) / FMHA_DECODE_ROWS;
+    const double n = (double)batch * p->nhead_k * (double)tiles;  // up to ~2^79
+    return n < 1e15 ? (int64_t)batch * p->nhead_k * tiles : (int64_t)1e15;
+}
+// Fills `a` but its workspace pointers for at most `chunks` key chunks per
+// (sequence, KV head), whole steps each; returns the workspace bytes.
+int64_t decode_plan(const FmhaFwdParams* p, int batch, int chunks, int64_t cus, FmhaDecodeArgs* a) {
+    const int steps = std::max(1, (p->seqlen_k + FMHA_DECODE_KEY_STEP - 1) / FMHA_DECODE_KEY_STEP);
+    const int per = (steps + chunks - 1) / chunks;
+    a->p = *p;
+    a->part = a->ml = nullptr;
+    a->chunk_keys = per * FMHA_DECODE_KEY_STEP;
+    a->n_chunks = (steps + per - 1) / per;
+    a->rows = (int)decode_rows(p);
+    const int64_t pairs = (int64_t)batch * p->nhead_k;
+    const int64_t blocks = pairs * a->n_chunks * ((a->rows + FMHA_DECODE_ROWS - 1) / FMHA_DECODE_ROWS);
+    // eight waves (one block per CU) halve a block's serial chain; short key
+    // ranges on more blocks than CUs take two four-wave blocks per CU, whose
+    // prologues and epilogues overlap (B64 H16/16 1 x 128: 14.9 / 10.8 us with
+    // 8 / 4 waves; 1 x 2048 on 320 blocks 36.2 / 34.7; 1 x 8000 varlen on 320
+    // 80.6 / 96.6)
+    a->waves = p->seqlen_k <= (blocks > cus ? 2048 : 128) ? 4 : 8;
+    return a->n_chunks == 1 ? 0 : pairs * a->n_chunks * a->rows * (FMHA_HEAD_DIM + 2) * (int64_t)sizeof(float);
+}
+// Key chunks of a launch with a workspace: none where the pairs fill half the
+// CUs (B16 H32/8 1 x 4100, 128 blocks: 28.7 us whole, 29.2 in two chunks; B64
+// H8/2 1 x 2048 13.4 / 16.2) or the chain is at most five steps (the merge
+// launch costs ~3 us, a step 0.6: B1 H8 4 x 4096, 16 steps, 15.7 whole, 9.8 in
+// eight chunks); else as many as fit the CUs in one round (12 sequences to
+// 16,000 keys, 24 pairs: 10 chunks 16.3 us, 16 chunks, a partial second round,
+// 19.7).
+int decode_chunks(const FmhaFwdParams* p, int batch, int64_t cus) {
+    const int64_t items = decode_items(p, batch);
+    if (items <= 0 || 2 * items >= cus || p->seqlen_k <= 5 * FMHA_DECODE_KEY_STEP) return 1;
+    return (int)std::min<int64_t>(FMHA_DECODE_MAX_CHUNKS, cus / items);
+}
+// Whether a launch runs it: the automatic choice without an order flag (those
+// ask for the M-tile grid); the bounds steer varlen launches.  Two regions:
+//  * decode proper, at most 32 queries (64 from 1024 keys) and 128 packed
+//    rows, bound by the K/V stream.  M-tile forms / decode, us, one box (dense
+//    caches, LSE): B16 H32/8 1 x 4100 82 / 28, B1 H32/8 1 x 32768 312 / 18, B2
+//    H16/2 16 x 16384 77 / 13, B64 H16/16 1 x 128 11.5 / 10.8, B16 H16/16 64 x
+//    4096 62 / 53; past 32 queries short key ranges lose (B64 H16 64 x 200
+//    17 / 22) and past 64 the M-tile forms win (B16 H16 128 x 4096 64 / 87: four
+//    row tiles re-read K and V).
+//  * dense launches of at most one 32-row tile per compute unit, bound by one
+//    block's chain of key tiles, which the decode form splits over eight waves:
+//    5.9 + 0.65 us per 256-key step (0.8 above half a block per CU, where two
+//    waves share a SIMD's matrix core with nothing left over) + 3.2 for the
+//    merge of a split launch, against the estimates of the other forms.  H8
+//    S512 8.0 / 6.9, H4 S1024 12.3 / 7.8, H8 S1024 causal 12.9 / 7.9, H2 S2048
+//    19.6 / 10.8, H4 256 x 8192 17.4 / 12.8, B8 H16/2 64 x 1000 13.2 / 8.3, H16
+//    100 x 8192 17.9 / 14.5 (chunks / decode); up to 256 keys both take one
+//    launch's latency (H2 S128 6.7 / 6.5 and 7.0 / 7.3 on two boxes) and the
+//    M-tile forms stay; H16/4 512 x 16384 stays in chunks (46 / 56).
+//
+// `split`: a workspace holds the split launch's partials; `workspace`: there
+// is one at all (the balanced and chunk forms' estimates count).
+struct DecodeAsk {
+    int seqlen_q, seqlen_k, nhead_q, nhead_k, batch, causal, split, workspace;
+    int64_t cus;
+    bool operator==(const DecodeAsk& o) const {
+        return seqlen_q == o.seqlen_q && seqlen_k == o.seqlen_k && nhead_q == o.nhead_q && nhead_k == o.nhead_k &&
+               batch == o.batch && causal == o.causal && split == o.split && workspace == o.workspace &&
+               cus == o.cus;
+    }
+};
+bool decode_faster(const FmhaFwdParams* p, const DecodeAsk& a) {
+    const int64_t items = decode_items(p, a.batch);
+    if (items > a.cus) return false;
+    const int chunks = a.split ? decode_chunks(p, a.batch, a.cus) : 1;
+    const int steps = (p->seqlen_k + FMHA_DECODE_KEY_STEP - 1) / FMHA_DECODE_KEY_STEP;
+    const double us =
+        5.9 + (2 * items > a.cus ? 0.8 : 0.65) * ((steps + chunks - 1) / chunks) + (chunks > 1 ? 3.2 : 0.0);
+    return us < 0.97 * mtile_us(p, a.batch, a.causal, a.cus, a.workspace != 0).us;
+}
+bool takes_decode(const FmhaFwdParams* p, int batch, int causal, int variant, bool split, bool workspace) {
+    if (variant != FMHA_VARIANT_AUTO || batch <= 0 || p->seqlen_q <= 0 || p->seqlen_k < 128) return false;
+    if (decode_rows(p) <= 128 && (p->seqlen_q <= 32 || (p->seqlen_q <= 64 && p->seqlen_k >= 1024))) return true;
+    if (p->seqstart_q != nullptr) return false;
+    // the estimates walk the M-tiles: a thread's last answer is kept (it
+    // depends on the shape only)
+    thread_local DecodeAsk last{-1, -1, -1, -1, -1, -1, -1, -1, -1};
+    thread_local bool last_answer = false;
+    const DecodeAsk ask{p->seqlen_q, p->seqlen_k, p->nhead_q, p->nhead_k, batch, causal,
+                        split, workspace, device_cus()};
+    if (!(ask == last)) {
+        last_answer = decode_faster(p, ask);
+        last = ask;
+    }
+    return last_answer;
+}
+
+hipError_t decode_launch(const FmhaDecodeArgs& a, int batch, int causal, hipStream_t stream) {
+    using Entry = void (*)(FmhaDecodeArgs);
+    static const Entry walk[2][2][2] = {
+        {{fmha_fwd_d64_bf16_decode_msk0, fmha_fwd_d64_bf16_decode_msk0_varlen},
+         {fmha_fwd_d64_bf16_decode_msk1, fmha_fwd_d64_bf16_decode_msk1_varlen}},
+        {{fmha_fwd_d64_bf16_decode4_msk0, fmha_fwd_d64_bf16_decode4_msk0_varlen},
+         {fmha_fwd_d64_bf16_decode4_msk1, fmha_fwd_d64_bf16_decode4_msk1_varlen}}};
+    static const Entry merge[2][2] = {
+        {fmha_fwd_d64_bf16_decode_merge_msk0, fmha_fwd_d64_bf16_decode_merge_msk0_varlen},
+        {fmha_fwd_d64_bf16_decode_merge_msk1, fmha_fwd_d64_bf16_decode_merge_msk1_varlen}};
+    const int c = causal ? 1 : 0, v = a.p.seqstart_q != nullptr ? 1 : 0;
+    hipLaunchKernelGGL(walk[a.waves == 4 ? 1 : 0][c][v],
+                       dim3(a.p.nhead_k * a.n_chunks, (a.rows + FMHA_DECODE_ROWS - 1) / FMHA_DECODE_ROWS, batch),
+                       dim3(64 * a.waves), 0, stream, a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || a.n_chunks == 1) return e;
+    hipLaunchKernelGGL(merge[c][v],
+                       dim3((a.rows + FMHA_DECODE_MERGE_ROWS - 1) / FMHA_DECODE_MERGE_ROWS, a.p.nhead_k, batch),
+                       dim3(64 * FMHA_DECODE_MERGE_ROWS), 0, stream, a);
+    return hipGetLastError();
+}
+// Workspace bytes of the split launch (0: never split).
+int64_t decode_bytes(const FmhaFwdParams* p, int batch) {
+    if (batch <= 0 || p->seqlen_q <= 0 || decode_items(p, batch) > INT32_MAX) return 0;
+    FmhaDecodeArgs a;
+    const int64_t cus = device_cus();
+    return decode_plan(p, batch, decode_chunks(p, batch, cus), cus, &a);
+}
+// The launch with as many chunks as the workspace holds: the plan's, or one.
+hipError_t decode_run(const FmhaFwdParams* p, int batch, int causal, void* workspace, int64_t workspace_bytes,
+                      hipStream_t stream) {
+    FmhaDecodeArgs a;
+    const int64_t cus = device_cus();
+    if (decode_plan(p, batch, decode_chunks(p, batch, cus), cus, &a) > workspace_bytes)
+        decode_plan(p, batch, 1, cus, &a);
+    if (a.n_chunks > 1) {
+        a.part = (float*)workspace;
+        a.ml = a.part + (int64_t)batch * p->nhead_k * a.n_chunks * a.rows * FMHA_HEAD_DIM;
+    }
+    return decode_launch(a, batch, causal, stream);
+}
+
+bool chunk_plan_build(const FmhaFwdParams* p, int batch, int causal, int64_t cus, FmhaChunkArgs* a, int64_t* bytes) {
+    const int m_tiles = (p->seqlen_q + kM0 - 1) / kM0;
+    if ((int64_t)p->nhead_q * batch > cus || (int64_t)p->nhead_q * batch * m_tiles > cus) return false;
+    const int tiles = mtile_us(p, batch, causal, cus, true).tiles;
+    if (tiles == 0) return false;
+    const int longest = mtile_tiles(p, causal, m_tiles - 1);
+    a->tiles = tiles;
+    a->max_chunks = std::min(FMHA_CHUNK_MAX_CHUNKS, chunk_count(longest, tiles));
+    // the heaviest M-tiles first, each one's chunks together
+    int n = 0, slots = 0;
+    unsigned short first[FMHA_CHUNK_MAX_MTILES];
+    for (int mt = m_tiles - 1; mt >= 0; --mt) {
+        const int nc = std::min(a->max_chunks, chunk_count(mtile_tiles(p, causal, mt), tiles));
+        if (n + nc + m_tiles > FMHA_CHUNK_TABLE) return false;
+        first[mt] = (unsigned short)slots;
+        slots += nc > 1 ? nc : 0;
+        for (int c = 0; c < nc; ++c) a->tab[n++] = (unsigned short)(mt << 6 | c);
+    }
+    std::copy(first, first + m_tiles, a->tab + n);
+    a->n_items = n;
+    a->n_slots = slots;
+    *bytes = (int64_t)batch * p->nhead_q * slots * FMHA_BALANCED_PART_BYTES;
+    return true;
+}
+// The plan of a launch with this variant (the automatic choice without an
+// order flag); fills `a` but its workspace pointer.  It depends on the shape
+// only, so the last one built on a thread is kept, as the balanced form's.
+bool chunk_plan(const FmhaFwdParams* p, int batch, int causal, int variant, FmhaChunkArgs* a, int64_t* bytes) {
+    if (variant != FMHA_VARIANT_AUTO || batch <= 0 || p->seqlen_q <= 0 || p->seqstart_q != nullptr) return false;
+    const int64_t cus = device_cus();
+    struct Key {
+        int seqlen_q, seqlen_k, nhead_q, batch, causal;
+        int64_t cus;
+        bool operator==(const Key& o) const {
+            return seqlen_q == o.seqlen_q && seqlen_k == o.seqlen_k && nhead_q == o.nhead_q && batch == o.batch &&
+                   causal == o.causal && cus == o.cus;
+        }
+    };
+    thread_local Key last_key{-1, -1, -1, -1, -1, -1};
+    thread_local bool last_ok = false;
+    thread_local int64_t last_bytes = 0;
+    thread_local FmhaChunkArgs last;
+    const Key key{p->seqlen_q, p->seqlen_k, p->nhead_q, batch, causal, cus};
+    if (!(key == last_key)) {
+        last_ok = chunk_plan_build(p, batch, causal, cus, &last, &last_bytes);
+        last_key = key;
+    }
+    if (!last_ok) return false;
+    *bytes = last_bytes;
+    if (a != nullptr) {
+        *a = last;
+        a->p = *p;
+    }
+    return true;
+}
+hipError_t chunk_launch(const FmhaChunkArgs& a, int batch, int causal, hipStream_t stream) {
+    const dim3 block(kBlockSize), walk(a.p.nhead_q, batch, a.n_items),
+        merge(a.p.nhead_q, 4 * ((a.p.seqlen_q + kM0 - 1) / kM0), batch);
+    if (causal)
+        hipLaunchKernelGGL(fmha_fwd_d64_bf16_chunk_msk1, walk, block, 0, stream, a);
+    else
+        hipLaunchKernelGGL(fmha_fwd_d64_bf16_chunk_msk0, walk, block, 0, stream, a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    if (causal)
+        hipLaunchKernelGGL(fmha_fwd_d64_bf16_chunk_balanced_merge_msk1, merge, block, 0, stream, a);
+    else
+        hipLaunchKernelGGL(fmha_fwd_d64_bf16_chunk_balanced_merge_msk0, merge, block, 0, stream, a);
+    return hipGetLastError();
+}
+
 // The plan mode of a variant that takes a workspace, or -1 for the others.
 int plan_mode(int v) {
     return v == FMHA_VARIANT_AUTO            ? kPlanAuto
@@ -540,7 +742,7 @@ int64_t fmha_balanced_workspace_size(const FmhaFwdParams* p, int batch, int caus
     if (order_of(variant) < 0) return -1;
     const int mode = plan_mode(variant & ~kOrderFlags);
     if (mode < 0) return 0;
-    if (takes_decode(p, variant)) return 0;
+    if (takes_decode(p, batch, causal, variant, false, false)) return 0;
     int64_t bytes = 0;
     // the same plan (and cache entry) as the launch with this variant
     const int xccs = order_of(variant) == kOrderReference ? 1 : device_shape().xccs;
@@ -549,11 +751,12 @@ int64_t fmha_balanced_workspace_size(const FmhaFwdParams* p, int batch, int caus
 }
 
 extern "C" int64_t fmha_fwd_d64_bf16_workspace_size(const FmhaFwdParams* p, int batch, int causal, int variant) {
-    const int64_t bytes = fmha_balanced_workspace_size(p, batch, causal, variant);
-    if (bytes != 0 || !takes_decode(p, variant)) return bytes;
-    FmhaDecodeArgs a;
-    const int64_t cus = device_cus();
-    return decode_plan(p, batch, decode_chunks(p, batch, cus), cus, &a);
+    const hipError_t chk = fmha_fwd_d64_bf16_check(p, batch, causal);
+    if (chk != hipSuccess) return -1;
+    int64_t bytes = 0;
+    if (takes_decode(p, batch, causal, variant, true, true)) return decode_bytes(p, batch);
+    if (chunk_plan(p, batch, causal, variant, nullptr, &bytes)) return bytes;
+    return fmha_balanced_workspace_size(p, batch, causal, variant);
 }
 
 extern "C" hipError_t fmha_fwd_d64_bf16_ws(const FmhaFwdParams* p, int batch, int causal, int variant,
@@ -567,7 +770,14 @@ extern "C" hipError_t fmha_fwd_d64_bf16_ws(const FmhaFwdParams* p, int batch, in
         (reinterpret_cast<uintptr_t>(workspace) & 255u))
         return hipErrorInvalidValue;
     if (batch == 0 || p->seqlen_q == 0) return hipSuccess;
-    if (takes_decode(p, variant)) return decode_run(p, batch, causal, workspace, workspace_bytes, stream);
+    if (takes_decode(p, batch, causal, variant, decode_bytes(p, batch) <= workspace_bytes, workspace_bytes > 0))
+        return decode_run(p, batch, causal, workspace, workspace_bytes, stream);
+    FmhaChunkArgs c;
+    int64_t chunk_bytes = 0;
+    if (chunk_plan(p, batch, causal, variant, &c, &chunk_bytes) && chunk_bytes <= workspace_bytes) {
+        c.part = (float*)workspace;
+        return chunk_launch(c, batch, causal, stream);
+    }
     FmhaBalancedArgs a;
     int64_t need = 0;
     // the reference-order flag keeps the plain heaviest-first table (the
@@ -600,7 +810,6 @@ extern "C" int fmha_fwd_d64_bf16_pick_variant(const FmhaFwdParams* p, int batch,
 extern "C" int fmha_fwd_d64_bf16_tile_major(const FmhaFwdParams* p, int batch, int causal) {
     if (fmha_fwd_d64_bf16_check(p, batch, causal) != hipSuccess) return -1;
     if (p->seqlen_q == 0 || batch == 0) return 0;  // nothing is launched
-    if (takes_decode(p, FMHA_VARIANT_AUTO)) return 0;
     if (dense_tile_major(p, batch, causal, kOrderAuto)) return 1;
     // varlen: the compact orders, which only the regular form has
     if (pick_form(p, batch, causal, device_cus()) != FMHA_VARIANT_REGULAR) return 0;
@@ -615,7 +824,7 @@ extern "C" hipError_t fmha_fwd_d64_bf16_variant(const FmhaFwdParams* p, int batc
     const int order = order_of(variant);
     if (order < 0) return hipErrorInvalidValue;  // more than one order flag
     const bool tile_major = dense_tile_major(p, batch, causal, order);
-    const bool decode = takes_decode(p, variant);
+    const bool decode = takes_decode(p, batch, causal, variant, false, false);
     variant &= ~kOrderFlags;
     // the balanced forms need fmha_fwd_d64_bf16_ws; 4 is a retired value
     if (!(variant == FMHA_VARIANT_AUTO || variant == FMHA_VARIANT_REGULAR || variant == FMHA_VARIANT_SPLITKV ||

@@ -129,20 +129,52 @@ struct Softmax {
 //  * kModeBalancedPair: kModePair's two groups on one item of a balanced
 //    causal launch of M-tile pairs: the pair's key tiles, or one half of
 //    them, each group's partial result to its own M-tile's slot.
-enum : int { kModeRegular = 0, kModeSplitKV = 1, kModePair = 2, kModeBalanced = 3, kModeBalancedPair = 4 };
+//  * kModeChunk: one group, one key chunk of an M-tile: M-tiles of more than
+//    `tiles` key tiles are cut into equal chunks, each leaving its partial
+//    result in its slot for the merge launch.
+enum : int {
+    kModeRegular = 0,
+    kModeSplitKV = 1,
+    kModePair = 2,
+    kModeBalanced = 3,
+    kModeBalancedPair = 4,
+    kModeChunk = 5
+};
 // The key range of a balanced-launch item: `part` null for a whole M-tile;
 // otherwise half `half` of its key tiles and the slot of its partial result.
+// Of a chunk launch: chunk `half` of the M-tile, in chunks of at most `tiles`
+// key tiles and at most `max` of them.
 struct Chunk {
     int half;
     float* part;
+    int tiles, max;
 };
+// Key tiles of an M-tile whose last row is `last` (pipeline.hpp:168-193).
+template <bool kCausal>
+__device__ __forceinline__ int key_tiles(int last, int sq, int sk) {
+    int kv_end = sk;
+    if constexpr (kCausal) {
+        const int e = min(last, sq - 1) + (sk - sq) + 1;
+        kv_end = e < 0 ? 0 : (e > sk ? sk : e);
+    }
+    return (kv_end + kTileN - 1) / kTileN;
+}
+// Chunks of an M-tile of n key tiles; chunk i holds tiles [chunk_start(i),
+// chunk_start(i + 1)).
+__device__ __forceinline__ int chunk_count(int n, int tiles, int max) {
+    return ::max(1, min(max, (n + tiles - 1) / tiles));
+}
+__device__ __forceinline__ int chunk_start(int i, int n, int count) {
+    return (int)(((unsigned)i * (unsigned)n + (unsigned)count - 1) / (unsigned)count);
+}
 template <bool kCausal, bool kVarlen, int kMode>
 __device__ __forceinline__ void fwd_mtile(const FmhaFwdParams& p, int b, int h, int mt, const Ring& ring,
-                                          Chunk ck = Chunk{0, nullptr}) {
-    constexpr int kGroups = (kMode == kModeRegular || kMode == kModeBalanced) ? 1 : 2;
+                                          Chunk ck = Chunk{0, nullptr, 0, 0}) {
+    constexpr int kGroups = (kMode == kModeRegular || kMode == kModeBalanced || kMode == kModeChunk) ? 1 : 2;
     constexpr bool kSplitKV = kMode == kModeSplitKV;
     constexpr bool kPair = kMode == kModePair || kMode == kModeBalancedPair;
-    constexpr bool kBalanced = kMode == kModeBalanced || kMode == kModeBalancedPair;
+    constexpr bool kChunk = kMode == kModeChunk;
+    constexpr bool kBalanced = kMode == kModeBalanced || kMode == kModeBalancedPair || kChunk;
     constexpr int kLoads = kPair ? 1 : kLoadsPerTile;  // DMA loads per wave, tensor and tile
     const int lane = threadIdx.x & 63;
     const int wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
@@ -207,7 +239,15 @@ __device__ __forceinline__ void fwd_mtile(const FmhaFwdParams& p, int b, int h, 
     // below count group-local tiles 0 .. ntg-1); tiles >= tile_end are dead
     int ntg = kSplitKV ? (ntiles + 1) / 2 : ntiles;
     int tile0 = kSplitKV ? group * ntg : 0;
-    if constexpr (kBalanced) {
+    if constexpr (kChunk) {
+        const int count = chunk_count(ntiles, ck.tiles, ck.max);
+        if (count > 1) {
+            tile0 = chunk_start(ck.half, ntiles, count);
+            ntg = chunk_start(ck.half + 1, ntiles, count) - tile0;
+        } else {
+            ck.part = nullptr;
+        }
+    } else if constexpr (kBalanced) {
         if (ck.part != nullptr) {  // a split M-tile (pair): the first ceil(n/2) key tiles, or the rest
             const int h0 = (ntiles + 1) / 2;
             tile0 = ck.half ? h0 : 0;
@@ -1723,9 +1763,9 @@ FMHA_STREAM_ATTRS void fmha_fwd_d64_bf16_pair_stream_msk1(FmhaStreamArgs args) {
 // split M-tiles. ----
 static_assert(FMHA_BALANCED_PART_BYTES == kWaves * kPartFloatsPerWave * 4, "partial slot size");
 __device__ __forceinline__ Chunk balanced_chunk(const FmhaBalancedArgs& a, int b, int h, int mt, int half) {
-    if (mt < a.split_from) return Chunk{0, nullptr};
+    if (mt < a.split_from) return Chunk{0, nullptr, 0, 0};
     const int64_t slot = ((int64_t)(b * a.p.nhead_q + h) * a.n_split + (mt - a.split_from)) * 2 + half;
-    return Chunk{half, a.part + slot * (kWaves * kPartFloatsPerWave)};
+    return Chunk{half, a.part + slot * (kWaves * kPartFloatsPerWave), 0, 0};
 }
 FMHA_ENTRY_ATTRS void fmha_fwd_d64_bf16_balanced_msk1(FmhaBalancedArgs args) {
     FMHA_RING(ring, kTileBytes)
@@ -1804,6 +1844,87 @@ __global__ __launch_bounds__(FMHA_KBLOCK) void fmha_fwd_d64_bf16_balanced_merge(
         const float lse2 = __builtin_log2f(l_tot) + m;  // -inf when l == 0
         p.lse[(int64_t)b * p.nhead_q * sq + (int64_t)h * sq + my_row] = lse2 * 0.69314718055994530942f;
     }
+}
+
+// ---- chunk entries (this build's own; no counterpart in the reference):
+// dense launches whose M-tiles are too few to fill the GPU but long.  Grid
+// (nhead_q, batch, n_items); item z of every (batch, head) comes from the
+// launcher's table (M-tile << 6 | chunk, heaviest first). ----
+__device__ __forceinline__ float* chunk_slot(const FmhaChunkArgs& a, int b, int h, int slot) {
+    return a.part + ((int64_t)(b * a.p.nhead_q + h) * a.n_slots + slot) * (kWaves * kPartFloatsPerWave);
+}
+template <bool kCausal>
+__device__ __forceinline__ void chunk_item(const FmhaChunkArgs& a, const Ring& ring) {
+    const int it = a.tab[blockIdx.z];
+    const int mt = it >> 6, c = it & 63;
+    const int b = blockIdx.y, h = blockIdx.x;
+    float* const slot = chunk_slot(a, b, h, a.tab[a.n_items + mt] + c);
+    fwd_mtile<kCausal, false, kModeChunk>(a.p, b, h, mt, ring, Chunk{c, slot, a.tiles, a.max_chunks});
+}
+FMHA_ENTRY_ATTRS void fmha_fwd_d64_bf16_chunk_msk0(FmhaChunkArgs args) {
+    FMHA_RING(ring, kTileBytes)
+    chunk_item<false>(args, ring);
+}
+FMHA_ENTRY_ATTRS void fmha_fwd_d64_bf16_chunk_msk1(FmhaChunkArgs args) {
+    FMHA_RING(ring, kTileBytes)
+    chunk_item<true>(args, ring);
+}
+
+// Merge of an M-tile's chunks (grid (nhead_q, 4 x M-tiles, batch)): a wave
+// takes 32 rows x 16 columns (8 of the 32 O^T registers of the wave that wrote
+// them, lane for lane: 256 contiguous bytes per load), four chunks' loads in
+// flight; latency bounds it, so the M-tile is spread over 16 waves.
+template <bool kCausal>
+__device__ __forceinline__ void chunk_merge(const FmhaChunkArgs& a) {
+    const FmhaFwdParams& p = a.p;
+    const int lane = threadIdx.x & 63;
+    const int l32 = lane & 31, hi = lane >> 5;
+    const int mt = blockIdx.y >> 2, wave = blockIdx.y & 3;
+    const int e0 = 8 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // first register
+    const int h = blockIdx.x, b = blockIdx.z;
+    const int sq = p.seqlen_q;
+    const int wrow0 = mt * kTileM + wave * kRowsPerWave, row = wrow0 + l32;
+    if (wrow0 >= sq) return;
+    const int n = chunk_count(key_tiles<kCausal>(mt * kTileM + kTileM - 1, sq, p.seqlen_k), a.tiles, a.max_chunks);
+    if (n == 1) return;  // written by its block
+    const float* w = chunk_slot(a, b, h, a.tab[a.n_items + mt]) + wave * kPartFloatsPerWave + lane;
+    constexpr int kStep = kWaves * kPartFloatsPerWave;
+    float m = kMaxSeed;
+#pragma unroll 8
+    for (int c = 0; c < n; ++c) m = fmaxf(m, w[c * kStep + 32 * 64]);
+    float l = 0.0f, acc[8] = {};
+#pragma unroll 4
+    for (int c = 0; c < n; ++c) {
+        const float* x = w + c * kStep;
+        const float al = __builtin_amdgcn_exp2f(x[32 * 64] - m);
+        l = __builtin_fmaf(al, x[33 * 64], l);
+#pragma unroll
+        for (int r = 0; r < 8; ++r) acc[r] = __builtin_fmaf(al, x[(e0 + r) * 64], acc[r]);
+    }
+    l = wave_sum_halves(l);
+    if (row >= sq) return;
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    // register 16 db + r is column 32 db + 8 (r / 4) + 4 h + r % 4
+    __bf16* o = (__bf16*)p.o + (int64_t)b * p.batch_stride_o + (int64_t)h * p.nhead_stride_o +
+                (int64_t)row * p.stride_o + 2 * e0 + 4 * hi;
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+        bf16x2 x0, x1;
+        x0[0] = (__bf16)(acc[4 * g + 0] * inv);
+        x0[1] = (__bf16)(acc[4 * g + 1] * inv);
+        x1[0] = (__bf16)(acc[4 * g + 2] * inv);
+        x1[1] = (__bf16)(acc[4 * g + 3] * inv);
+        *(i32x2*)(o + 8 * g) = i32x2{__builtin_bit_cast(int, x0), __builtin_bit_cast(int, x1)};
+    }
+    if (p.lse != nullptr && hi == 0 && e0 == 0)
+        p.lse[((int64_t)b * p.nhead_q + h) * sq + row] =
+            (__builtin_log2f(l) + m) * 0.69314718055994530942f;  // -inf when l == 0
+}
+__global__ __launch_bounds__(FMHA_KBLOCK) void fmha_fwd_d64_bf16_chunk_balanced_merge_msk0(FmhaChunkArgs args) {
+    chunk_merge<false>(args);
+}
+__global__ __launch_bounds__(FMHA_KBLOCK) void fmha_fwd_d64_bf16_chunk_balanced_merge_msk1(FmhaChunkArgs args) {
+    chunk_merge<true>(args);
 }
 
 // ---- short entries (this build's own; no counterpart in the reference):

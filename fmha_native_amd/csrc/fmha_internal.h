@@ -24,6 +24,27 @@ __global__ void fmha_fwd_d64_bf16_balanced_msk1(FmhaBalancedArgs args);
 __global__ void fmha_fwd_d64_bf16_balanced_pair_msk1(FmhaBalancedArgs args);
 __global__ void fmha_fwd_d64_bf16_balanced_merge(FmhaBalancedArgs args);
 
+// Chunk form (see fmha_fwd_kernel.hip): long M-tiles cut into key chunks, on
+// dense grids whose M-tiles are too few to fill the GPU.
+#define FMHA_CHUNK_TABLE 1920
+#define FMHA_CHUNK_MAX_MTILES 1024 // 10 bits of an item
+#define FMHA_CHUNK_MAX_CHUNKS 64   // 6 bits
+struct FmhaChunkArgs {
+    FmhaFwdParams p;
+    float* part;     // partial results (FMHA_BALANCED_PART_BYTES each), n_slots per (batch, head)
+    int tiles;       // key tiles a chunk may hold
+    int max_chunks;  // chunks an M-tile may have
+    int n_items;     // items per (batch, head) (the grid's z)
+    int n_slots;     // slots per (batch, head)
+    // n_items items in dispatch order (M-tile << 6 | chunk), then every M-tile's
+    // first slot
+    unsigned short tab[FMHA_CHUNK_TABLE];
+};
+__global__ void fmha_fwd_d64_bf16_chunk_msk0(FmhaChunkArgs args);
+__global__ void fmha_fwd_d64_bf16_chunk_msk1(FmhaChunkArgs args);
+__global__ void fmha_fwd_d64_bf16_chunk_balanced_merge_msk0(FmhaChunkArgs args);
+__global__ void fmha_fwd_d64_bf16_chunk_balanced_merge_msk1(FmhaChunkArgs args);
+
 // Pair stream form (see fmha_fwd_kernel.hip): one 8-wave pair block per
 // compute unit looping over a static list of M-tile pairs.
 struct FmhaStreamArgs {
@@ -38,7 +59,6 @@ __global__ void fmha_fwd_d64_bf16_pair_stream_msk1(FmhaStreamArgs args);
 // key chunks.
 #define FMHA_DECODE_ROWS 32                            // packed rows (query heads of a KV head x tokens) per block
 #define FMHA_DECODE_KEY_STEP 256                       // keys eight waves take per step; chunks are multiples of it
-#define FMHA_DECODE_MAX_ROWS 128                       // packed rows per KV head a launch may have
 #define FMHA_DECODE_MAX_CHUNKS 64                      // the merge holds one chunk's weight per lane
 #define FMHA_DECODE_MERGE_ROWS 4                       // rows (waves) per merge block
 struct FmhaDecodeArgs {

@@ -115,9 +115,11 @@ hipError_t fmha_fwd_d64_bf16(const FmhaFwdParams* params, int batch, int causal,
 /* The same launch with the kernel form chosen by the caller (this build's
  * own; no counterpart in the reference):
  *   FMHA_VARIANT_AUTO     what fmha_fwd_d64_bf16() picks: the decode form (below)
- *                         for at most 32 queries (64 from 1024 keys on), at
- *                         most 128 rows per KV head (nhead_q / nhead_k x
- *                         seqlen_q), seqlen_k >= 128 and no order flag; short for
+ *                         from 128 keys on for at most 32 queries (64 from
+ *                         1024 keys on) and 128 rows per KV head (nhead_q /
+ *                         nhead_k x seqlen_q), and for dense launches of at most
+ *                         CUs x 32 such rows in all where it is estimated
+ *                         faster; short for
  *                         launches with seqlen_k <= 192 and at least
  *                         2 x CUs x 128 query rows (batch x nhead_q x
  *                         seqlen_q; varlen: the bounds), or causal with
@@ -148,7 +150,8 @@ hipError_t fmha_fwd_d64_bf16(const FmhaFwdParams* params, int batch, int causal,
  *                         taking that pair's mirror next
  * The decode form has no code of its own: the query heads of a KV head share
  * one pass over its keys, whose 32-key steps the waves of a block split, and
- * with a workspace (fmha_fwd_d64_bf16_ws) the blocks too.  In varlen launches
+ * with a workspace (fmha_fwd_d64_bf16_ws) the blocks too; an order flag keeps
+ * the M-tile forms.  In varlen launches
  * seqlen_q must bound every sequence's queries (rows past it are not
  * computed); seqlen_k only steers the choice and the split.
  * All forms give the same results up to fp32 rounding order.  Causal dense
@@ -202,7 +205,11 @@ hipError_t fmha_fwd_d64_bf16_variant(const FmhaFwdParams* params, int batch, int
  *            blocks where the (sequence, KV head) pairs fill less than half
  *            the compute units and seqlen_k > 1280: each block's fp32 partial
  *            goes to the workspace and a second launch merges them, unsplit
- *            if the workspace is too small; else what fmha_fwd_d64_bf16 picks),
+ *            if the workspace is too small; the chunk form for dense launches
+ *            of at most 0.6 M-tiles per compute unit whose long M-tiles it
+ *            estimates faster in key chunks: each chunk's fp32 partial goes to
+ *            the workspace and a second launch merges them; without an order
+ *            flag; else what fmha_fwd_d64_bf16 picks),
  *            FMHA_VARIANT_BALANCED (always the balanced form, with the
  *            heavy-M-tile rule applied even where the regular order would
  *            balance: causal dense only; hipErrorInvalidValue if it cannot
@@ -275,7 +282,8 @@ int fmha_fwd_d64_bf16_pick_variant(const FmhaFwdParams* params, int batch, int c
  * with these arguments: 1 for a tile-major entry (causal dense batches) or the
  * level order of a compact varlen entry, 2 for the sequence order of a
  * compact varlen entry, 0 for the reference's order, -1 for rejected
- * arguments; host only (this build's own; no counterpart in the reference). */
+ * arguments (of the M-tile form, where the decode or chunk form does not take
+ * the launch); host only (this build's own; no counterpart in the reference). */
 int fmha_fwd_d64_bf16_tile_major(const FmhaFwdParams* params, int batch, int causal);
 
 /* Tile constants of the linked library, so FFI callers (ctypes, cgo) need not

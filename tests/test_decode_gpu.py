@@ -62,18 +62,22 @@ def test_decode_split_rule(h, hk, sq, sk, batch, chunks):
     assert fmha.workspace_size(p, batch, 0, fmha.VARIANT_REFERENCE_ORDER) == 0
 
 
-@pytest.mark.parametrize("h,hk,sq,sk", [(32, 8, 33, 4096), (8, 8, 65, 4096), (8, 8, 33, 1023), (8, 8, 0, 4096)])
-def test_decode_leaves_other_launches(h, hk, sq, sk):
-    """More than 128 rows, more than 64 queries or more than 32 over fewer
-    than 1024 keys: the M-tile forms (dense: no workspace)."""
-    assert fmha.workspace_size(_params(h, hk, sq, sk), 1, 0) == 0
+@pytest.mark.parametrize("b,h,hk,sq,sk,decode", [
+    (1, 16, 16, 100, 8192, True), (1, 1, 1, 200, 9000, True), (2, 8, 1, 64, 3000, True),  # one row tile per CU at most
+    (16, 16, 16, 100, 8192, False), (1, 16, 4, 512, 16384, False), (1, 8, 8, 0, 4096, False)])
+def test_decode_takes_small_launches(b, h, hk, sq, sk, decode):
+    """Past 128 rows or 64 queries: where one 32-row tile per compute unit
+    holds the launch and the estimates say so (seen in the workspace: the
+    M-tile forms' are whole 34,816-byte partial results)."""
+    assert (fmha.workspace_size(_params(h, hk, sq, sk), b, 0) % 34816 != 0) == decode
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("causal", [0, 1])
 @pytest.mark.parametrize("b,h,hk,sq,sk", [
     (3, 8, 2, 1, 128), (2, 16, 2, 4, 255), (1, 3, 3, 31, 257), (40, 16, 16, 2, 300),   # 640 pairs: four-wave blocks
-    (1, 8, 2, 1, 1281), (2, 32, 4, 16, 4100), (1, 2, 2, 64, 5000), (1, 8, 1, 7, 20011), (20, 32, 8, 1, 2048)])
+    (1, 8, 2, 1, 1281), (2, 32, 4, 16, 4100), (1, 2, 2, 64, 5000), (1, 8, 1, 7, 20011), (20, 32, 8, 1, 2048),
+    (1, 4, 4, 512, 512), (1, 6, 3, 1000, 1000), (2, 2, 1, 700, 701), (1, 2, 2, 2049, 2047), (1, 1, 1, 200, 9000)])
 def test_decode_matches_float64(b, h, hk, sq, sk, causal):
     """Whole and split, from a KV cache whose tail is NaN and with O and LSE
     poisoned; the split launch twice on a dirty workspace (equal bits)."""
