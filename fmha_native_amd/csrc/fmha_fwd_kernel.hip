@@ -77,8 +77,11 @@ struct Ring {
 // exp, 32 add, 16 cvt_pk, bookkeeping) lands as 8-11 per slot over the first
 // 12 slots and the last GEMM0 chain runs bare.  A rigid even spread (every
 // slot fenced with sched_barrier, 7 VALU each) gives the same bits and is
-// 2-3% slower on the benchmark grids.
-constexpr int kValuPerSlot = 7;
+// 2-3% slower on the benchmark grids.  Five VALU per slot leaves the scheduler
+// more of them to place than seven: causal B1 H16 S8192 145.8 -> 142.4 us, B4 H16
+// S2048 73.0 -> 71.3, eight packed causal sequences H16 126.6 -> 122.7 (3 and 4
+// within 0.5 % of 5; reads four MFMAs ahead instead of two within 1 %).
+constexpr int kValuPerSlot = 5;
 constexpr int kDsAhead = 2;
 template <bool kG1, bool kG0>
 struct IterSchedule {
