@@ -712,6 +712,42 @@ hipError_t chunk_launch(const FmhaChunkArgs& a, int batch, int causal, hipStream
     return hipGetLastError();
 }
 
+// Whether the automatic choice takes the wide form (64 rows per wave, 256 per
+// block): dense layouts whose M-tile form would be the regular or the pair form.
+//  * Blocks of about equal work (no mask, or a causal key range much longer
+//    than the queries): a CU with two blocks takes 1.86 us per key tile of both
+//    and one block alone 1.08 (regular 1.12 and 0.60 for half the rows, pair
+//    1.065), so with k blocks on the fullest CU the launch takes 1.86 (k / 2) +
+//    1.08 (k % 2) us per key tile, and the estimates are compared.  Over 26
+//    shapes (S256-S8192, 192-3,072 blocks, us, other / wide): k = 2 B4 H16 S2048
+//    71 / 65, B64 H8 S256 17.2 / 15.5; k = 3 full B6 H16 S2048 108 / 98, B12 H16
+//    S1000 58 / 52; partial last rounds lose: B3 H16 S2048 (1.5 rounds) 56 / 60,
+//    B9 H16 S900 43.6 / 44.9, B8 H16 S1030 (an odd M-tile) 47.1 / 48.5.
+//  * Causal squares: the heaviest-first order levels the blocks from four per CU,
+//    and the waves' different diagonals (up to three tiles of a block's) cost
+//    little from 2,560 keys: H32 S8192 283 / 262, H16 S16384 543 / 501, B12 H32
+//    S3000 519 / 478, B4 H32 S4096 304 / 290; B16 H16 S2048 179 / 178, B16 H16
+//    S1024 56 / 63, H24 S6000 (576 blocks) 122 / 130, H16 S8192 (512) 142 / 155.
+bool takes_wide(const FmhaFwdParams* p, int batch, int causal, int variant, int64_t cus) {
+    if (variant != FMHA_VARIANT_AUTO || p->seqstart_q != nullptr || batch <= 0 || p->seqlen_q <= 0 ||
+        p->seqlen_k <= 0)
+        return false;
+    const int form = pick_form(p, batch, causal, cus);
+    if (form != FMHA_VARIANT_REGULAR && form != FMHA_VARIANT_PAIR) return false;
+    const int m_tiles = (p->seqlen_q + kM0 - 1) / kM0;
+    const int longest = mtile_tiles(p, causal, m_tiles - 1);
+    const int lightest = mtile_tiles(p, causal, std::min(1, m_tiles - 1));
+    const int64_t wide = pair_blocks(p, batch), regular = grid_blocks(p, batch);
+    if (4 * (int64_t)lightest < 3 * (int64_t)longest) return wide >= 4 * cus && longest >= 40;
+    auto us = [cus](int64_t blocks, double two, double one) {
+        const int64_t k = (blocks + cus - 1) / cus;  // blocks of the fullest CU
+        return two * (double)(k / 2) + one * (double)(k % 2);
+    };
+    double other = us(regular, 1.12, 0.60);
+    if (form == FMHA_VARIANT_PAIR) other = std::min(other, 1.065 * (double)(wide / cus));
+    return us(wide, 1.86, 1.08) < 0.97 * other;
+}
+
 // The plan mode of a variant that takes a workspace, or -1 for the others.
 int plan_mode(int v) {
     return v == FMHA_VARIANT_AUTO            ? kPlanAuto
@@ -854,6 +890,19 @@ extern "C" hipError_t fmha_fwd_d64_bf16_variant(const FmhaFwdParams* p, int batc
         else
             hipLaunchKernelGGL(fmha_fwd_d64_bf16_pair_stream_msk0, dim3((unsigned)blocks), dim3(FMHA_SPLIT_KBLOCK), 0,
                                stream, a);
+        return hipGetLastError();
+    }
+    if (order == kOrderAuto && takes_wide(p, batch, causal, variant, device_cus())) {
+        const int blocks = (m_tiles + 1) / 2;
+        if (tile_major)
+            hipLaunchKernelGGL(fmha_fwd_d64_bf16_wide_msk1_tilemajor, dim3(p->nhead_q, batch, blocks), dim3(kBlockSize),
+                               0, stream, *p);
+        else if (causal)
+            hipLaunchKernelGGL(fmha_fwd_d64_bf16_wide_msk1, dim3(p->nhead_q, blocks, batch), dim3(kBlockSize), 0,
+                               stream, *p);
+        else
+            hipLaunchKernelGGL(fmha_fwd_d64_bf16_wide_msk0, dim3(p->nhead_q, blocks, batch), dim3(kBlockSize), 0,
+                               stream, *p);
         return hipGetLastError();
     }
     if (variant == FMHA_VARIANT_AUTO)

@@ -1650,6 +1650,364 @@ __device__ __forceinline__ bool sequence_item(const FmhaFwdParams& p, int rank, 
     return true;
 }
 
+// ===========================================================================
+// Wide form (this build's own; no counterpart in the reference): 64 query rows
+// per wave, 256 per block of four waves, two blocks per compute unit.
+//
+// The tile pipeline of fwd_mtile is bound by VALU and MFMA issue at the chip's
+// power cap, and a wave of 32 rows pays one LDS operand read per MFMA and one
+// 8 KiB K and V tile of LDS-DMA per 128 rows.  Two 32-row blocks of queries per
+// wave share every K and V operand read (half the LDS reads per MFMA) and every
+// tile (half the DMA).  To fit 256 registers the pipeline steps by 32 keys:
+// step (t, half) issues GEMM1 of the step before, GEMM0 of the step after (8
+// MFMAs each) and the softmax of its own 32 x 64 scores, so its live state is
+// O^T 64 + Q 32 + scores 64 + P 32 registers (230 in all); the ring still moves
+// 64-key tiles, one barrier each, K(t+3) and V(t+2) in flight.
+// Measured against the form it replaces: B4 H16 S2048 71.2 -> 65.2 us (1,054
+// TFLOP/s), B8 H16 S1024 38.6 -> 35.2, B16 H16 S512 23.1 -> 20.8, H16 S8192 266
+// -> 246, B32 H32 S700 174 -> 151, causal H32 S8192 283 -> 262.
+// ===========================================================================
+constexpr int kWideValuPerSlot = 5;  // 7: 3 % slower, 3: 1 %
+constexpr int kWideDsAhead = 4;      // operand reads run this many MFMAs ahead (two per read); 2: within 1 %
+// Slots of one step: {1 MFMA, the reads of the MFMA kWideDsAhead later, VALU};
+// MFMAs 0-7 are GEMM1's (two tr_b16 reads per two MFMAs), 8-15 GEMM0's (one b128
+// read per two).
+struct WideSchedule {
+    static constexpr int reads(int m) { return m >= 16 || (m & 1) ? 0 : m < 8 ? 2 : 1; }
+    template <int I, bool kG1>
+    static __device__ __forceinline__ void slot() {
+        constexpr int kFirst = kG1 ? 0 : 8;
+        __builtin_amdgcn_sched_group_barrier(kSchedMFMA, 1, 0);
+        if constexpr (reads(I + kFirst + kWideDsAhead) > 0)
+            __builtin_amdgcn_sched_group_barrier(kSchedDSRead, reads(I + kFirst + kWideDsAhead), 0);
+        __builtin_amdgcn_sched_group_barrier(kSchedVALU, kG1 ? kWideValuPerSlot : 2 * kWideValuPerSlot, 0);
+    }
+    template <bool kG1, int... Is>
+    static __device__ __forceinline__ void run(std::integer_sequence<int, Is...>) {
+        __builtin_amdgcn_sched_group_barrier(kSchedDSRead, (kG1 ? 2 : 1) * (kWideDsAhead / 2), 0);
+        (slot<Is, kG1>(), ...);
+    }
+    template <bool kG1>
+    static __device__ __forceinline__ void apply() {
+        run<kG1>(std::make_integer_sequence<int, kG1 ? 16 : 8>{});
+    }
+};
+// Block `pr` of (b, h): rows 256 pr .. +255 (the pair form's two M-tiles).
+template <bool kCausal>
+__device__ __forceinline__ void fwd_wide(const FmhaFwdParams& p, int b, int h, int pr, const Ring& ring) {
+    constexpr int kRowsW = 64;
+    constexpr int kLoads = kLoadsPerTile;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l32 = lane & 31, hi = lane >> 5;
+    const int sq = p.seqlen_q, sk = p.seqlen_k;
+    const int blk_row0 = pr * 2 * kTileM;
+    const int kvh = h / (p.nhead_q / p.nhead_k);
+    const __bf16* qbase = (const __bf16*)p.q + (int64_t)b * p.batch_stride_q + (int64_t)h * p.nhead_stride_q;
+    const __bf16* kbase = (const __bf16*)p.k + (int64_t)b * p.batch_stride_k + (int64_t)kvh * p.nhead_stride_k;
+    const __bf16* vbase = (const __bf16*)p.v + (int64_t)b * p.batch_stride_v + (int64_t)kvh * p.nhead_stride_v;
+    __bf16* obase = (__bf16*)p.o + (int64_t)b * p.batch_stride_o + (int64_t)h * p.nhead_stride_o;
+    const uint32_t qbytes = sq > 0 ? (uint32_t)((int64_t)(sq - 1) * p.stride_q * 2 + kRowBytes) : 0u;
+    const uint32_t kbytes = sk > 0 ? (uint32_t)((int64_t)(sk - 1) * p.stride_k * 2 + kRowBytes) : 0u;
+    const uint32_t vbytes = sk > 0 ? (uint32_t)((int64_t)(sk - 1) * p.stride_v * 2 + kRowBytes) : 0u;
+    const uint32_t obytes = (uint32_t)((int64_t)(sq - 1) * p.stride_o * 2 + kRowBytes);
+    const int shift = sk - sq;
+    const int ntiles = key_tiles<kCausal>(blk_row0 + 2 * kTileM - 1, sq, sk);
+    const int wrow0 = blk_row0 + wave * kRowsW;
+    bf16x8 qop[2][4];
+
+    const int ld_row = (kLoads * wave) * 8 + (lane >> 3);
+    const int ld_pc = lane & 7;
+    const int k_ld_off0 = ld_row * p.stride_k * 2 + ((ld_pc ^ k_swz(ld_row)) << 4);
+    const int k_ld_off1 = (ld_row + 8) * p.stride_k * 2 + ((ld_pc ^ k_swz(ld_row + 8)) << 4);
+    const int v_ld_off0 = ld_row * p.stride_v * 2 + ((ld_pc ^ v_swz(ld_row)) << 4);
+    const int v_ld_off1 = (ld_row + 8) * p.stride_v * 2 + ((ld_pc ^ v_swz(ld_row + 8)) << 4);
+    const int k_tile_step = kTileN * p.stride_k * 2;
+    const int v_tile_step = kTileN * p.stride_v * 2;
+    const int wave_off = (kLoads * wave) * 1024;
+    auto issue_k = [&](int tile, auto stage_c) {
+        lds_char* dst = ring.k[decltype(stage_c)::value] + wave_off;
+        const uint32_t t0 = (uint32_t)tile * (uint32_t)k_tile_step;
+        const auto r = make_rsrc((const char*)kbase + t0, tile < ntiles ? kbytes - t0 : 0u);
+        lds_dma_16(r, dst, k_ld_off0);
+        lds_dma_16(r, dst + 1024, k_ld_off1);
+    };
+    auto issue_v = [&](int tile, auto stage_c) {
+        lds_char* dst = ring.v[decltype(stage_c)::value] + wave_off;
+        const uint32_t t0 = (uint32_t)tile * (uint32_t)v_tile_step;
+        const auto r = make_rsrc((const char*)vbase + t0, tile < ntiles ? vbytes - t0 : 0u);
+        lds_dma_16(r, dst, v_ld_off0);
+        lds_dma_16(r, dst + 1024, v_ld_off1);
+    };
+    uint32_t k_rd[4], v_rd[2];
+    {
+        const int f = k_swz(l32);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) k_rd[t] = l32 * kRowBytes + (((2 * t + hi) ^ f) << 4);
+        const int g = lane >> 4, i16 = lane & 15;
+        const int row = 4 * hi + (i16 >> 2), c = i16 & 3;
+#pragma unroll
+        for (int db = 0; db < 2; ++db) {
+            const int chunk = 4 * db + 2 * (g & 1) + (c >> 1);
+            v_rd[db] = row * kRowBytes + ((chunk ^ v_swz(row)) << 4) + (c & 1) * 8;
+        }
+    }
+    const float scale = p.scale;
+    const float scale_v = in_vgpr(scale);
+    float m_ref[2] = {kMaxSeed, kMaxSeed}, l_part[2] = {0.0f, 0.0f}, l_tile[2];
+    f32x16 oacc[2][2];  // [qb][db]
+#pragma unroll
+    for (int qb = 0; qb < 2; ++qb)
+#pragma unroll
+        for (int db = 0; db < 2; ++db) oacc[qb][db] = f32x16{};
+
+    auto gemm0 = [&](auto ks_c, int half, f32x16* s) {
+        const lds_char* st = ring.k[decltype(ks_c)::value] + half * 32 * kRowBytes;
+        f32x16 acc[2] = {f32x16{}, f32x16{}};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const bf16x8 a = lds_read_b128(st + k_rd[k]);
+#pragma unroll
+            for (int qb = 0; qb < 2; ++qb) acc[qb] = mfma(a, qop[qb][k], acc[qb]);
+        }
+        s[0] = acc[0];
+        s[1] = acc[1];
+    };
+    auto gemm1 = [&](auto vs_c, int half, const bf16x8* pp) {
+        const lds_char* st = ring.v[decltype(vs_c)::value] + half * 32 * kRowBytes;
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+            for (int db = 0; db < 2; ++db) {
+                const bf16x8 a = lds_read_vt(st + v_rd[db] + 16 * k * kRowBytes);
+#pragma unroll
+                for (int qb = 0; qb < 2; ++qb) oacc[qb][db] = mfma(a, pp[2 * qb + k], oacc[qb][db]);
+            }
+    };
+    auto mask_half = [&](int t, int half, f32x16* s) {
+        const int key0 = t * kTileN + 32 * half;
+        const bool need = (key0 + 32 > sk) || (kCausal && key0 + 31 > wrow0 + shift);
+        if (need) {
+            const float ninf = in_vgpr(-__builtin_inff());
+#pragma unroll
+            for (int qb = 0; qb < 2; ++qb) {
+                const int lim = kCausal ? min(sk - 1, wrow0 + 32 * qb + l32 + shift) : sk - 1;
+                const int d = lim - (key0 + 4 * hi);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) s[qb][r] = (8 * (r >> 2) + (r & 3)) <= d ? s[qb][r] : ninf;
+            }
+        }
+    };
+    auto half_max = [&](const f32x16& s) {
+        float mx = fmaxf(s[0], s[1]);
+#pragma unroll
+        for (int r = 2; r < 16; r += 2) mx = fmaxf(fmaxf(mx, s[r]), s[r + 1]);
+        return wave_max_halves(mx);
+    };
+    auto exp_half = [&](const f32x16* s, bf16x8* pp) {
+#pragma unroll
+        for (int qb = 0; qb < 2; ++qb) {
+            const float neg_ms = -m_ref[qb];
+            float ls[2];
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                bf16x8 pk;
+                float acc;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(s[qb][8 * k + e], scale_v, neg_ms));
+                    acc = e == 0 ? pv : acc + pv;
+                    pk[e] = (__bf16)pv;
+                }
+                ls[k] = acc;
+                pp[2 * qb + k] = pk;
+            }
+            l_tile[qb] = ls[0] + ls[1];
+        }
+    };
+    auto softmax = [&](const f32x16* s, bf16x8* pp) {
+        exp_half(s, pp);
+        asm volatile("" ::"v"(pp[0]), "v"(pp[1]), "v"(pp[2]), "v"(pp[3]), "v"(l_tile[0]), "v"(l_tile[1]));
+    };
+    auto settle = [&](const f32x16* s, bf16x8* pp) {
+        // as fwd_mtile's settle(), over both query blocks (the sums are >= 0)
+        if (__builtin_amdgcn_ballot_w64(!(l_tile[0] + l_tile[1] <= kGrowSum))) {
+            asm volatile("" ::: "memory");  // keeps the rare path a branch
+#pragma unroll
+            for (int qb = 0; qb < 2; ++qb) {
+                const float m_new = fmaxf(m_ref[qb], half_max(s[qb]) * scale);
+                const float alpha = __builtin_amdgcn_exp2f(m_ref[qb] - m_new);
+                m_ref[qb] = m_new;
+#pragma unroll
+                for (int db = 0; db < 2; ++db)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) oacc[qb][db][r] *= alpha;
+                l_part[qb] *= alpha;
+            }
+            exp_half(s, pp);
+        }
+        l_part[0] += l_tile[0];
+        l_part[1] += l_tile[1];
+    };
+    f32x16 sacc[2][2];
+    bf16x8 pbuf[2][4];
+    using P0 = std::integral_constant<int, 0>;
+    using P1 = std::integral_constant<int, 1>;
+    using P2 = std::integral_constant<int, 2>;
+    using P3 = std::integral_constant<int, 3>;
+    auto sync_issue = [&](int t, auto phase_c) {
+        constexpr int J = decltype(phase_c)::value;
+        vmcnt_wait<2 * kLoads>();
+        ring_barrier();
+        issue_k(t + 3, std::integral_constant<int, (J + 3) % kRing>{});
+        issue_v(t + 2, std::integral_constant<int, (J + 2) % kRing>{});
+    };
+    auto tile = [&](int t, auto phase_c, auto first_c) {
+        constexpr int J = decltype(phase_c)::value;
+        constexpr bool kFirst = decltype(first_c)::value;
+        sync_issue(t, phase_c);
+        mask_half(t, 0, sacc[0]);
+        if constexpr (!kFirst) gemm1(std::integral_constant<int, (J + 3) % kRing>{}, 1, pbuf[1]);
+        gemm0(std::integral_constant<int, J>{}, 1, sacc[1]);
+        softmax(sacc[0], pbuf[0]);
+        WideSchedule::apply<!kFirst>();
+        settle(sacc[0], pbuf[0]);
+        __builtin_amdgcn_sched_barrier(0);
+        mask_half(t, 1, sacc[1]);
+        gemm1(std::integral_constant<int, J>{}, 0, pbuf[0]);
+        gemm0(std::integral_constant<int, (J + 1) % kRing>{}, 0, sacc[0]);
+        softmax(sacc[1], pbuf[1]);
+        WideSchedule::apply<true>();
+        settle(sacc[1], pbuf[1]);
+    };
+    int nlive = ntiles;
+    if constexpr (kCausal) {
+        const int last_key = min(sk - 1, wrow0 + kRowsW - 1 + shift);
+        const int lt = last_key < 0 || wrow0 >= sq ? 0 : last_key / kTileN + 1;
+        nlive = max(1, min(ntiles, lt));
+    }
+    if (!kCausal && ntiles > 0 && wrow0 >= sq) {  // no rows: the ring only, as in fwd_mtile
+        issue_k(0, P0{});
+        issue_k(1, P1{});
+        issue_v(0, P0{});
+        issue_k(2, P2{});
+        issue_v(1, P1{});
+        vmcnt_wait<4 * kLoads>();
+        ring_barrier();
+        for (int t = 0; t < ntiles; t += kRing) {
+            sync_issue(t, P0{});
+            if (t + 1 >= ntiles) break;
+            sync_issue(t + 1, P1{});
+            if (t + 2 >= ntiles) break;
+            sync_issue(t + 2, P2{});
+            if (t + 3 >= ntiles) break;
+            sync_issue(t + 3, P3{});
+        }
+        vmcnt_wait<0>();
+        ring_barrier();
+        return;
+    }
+    if (ntiles > 0) {
+        const auto rq = make_rsrc(qbase, qbytes);
+#pragma unroll
+        for (int qb = 0; qb < 2; ++qb) {
+            const int qoff = (wrow0 + 32 * qb + l32) * p.stride_q * 2 + hi * 16;
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                qop[qb][t] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rq, qoff + t * 32, 0, 0));
+        }
+        issue_k(0, P0{});
+        issue_k(1, P1{});
+        issue_v(0, P0{});
+        issue_k(2, P2{});
+        issue_v(1, P1{});
+        vmcnt_wait<4 * kLoads>();
+        ring_barrier();
+        asm volatile("" ::"v"(qop[0][0]), "v"(qop[0][1]), "v"(qop[0][2]), "v"(qop[0][3]), "v"(qop[1][0]),
+                     "v"(qop[1][1]), "v"(qop[1][2]), "v"(qop[1][3]));
+        gemm0(P0{}, 0, sacc[0]);
+        mask_half(0, 0, sacc[0]);
+        m_ref[0] = fmaxf(kMaxSeed, half_max(sacc[0][0]) * scale);
+        m_ref[1] = fmaxf(kMaxSeed, half_max(sacc[0][1]) * scale);
+        tile(0, P0{}, std::true_type{});
+        int t = 1;
+        for (; t + kRing <= nlive; t += kRing) {
+            tile(t, P1{}, std::false_type{});
+            tile(t + 1, P2{}, std::false_type{});
+            tile(t + 2, P3{}, std::false_type{});
+            tile(t + 3, P0{}, std::false_type{});
+        }
+        const int rem = nlive - t;
+        if (rem >= 1) tile(t, P1{}, std::false_type{});
+        if (rem >= 2) tile(t + 1, P2{}, std::false_type{});
+        if (rem >= 3) tile(t + 2, P3{}, std::false_type{});
+        // the last live tile's (phase rem) second-half GEMM1 after the next
+        // barrier, then the ring goes on without compute
+        auto finish = [&](auto phase_c) {
+            constexpr int J = decltype(phase_c)::value;
+            if (kCausal && nlive < ntiles) {
+                sync_issue(nlive, std::integral_constant<int, (J + 1) % kRing>{});
+                gemm1(phase_c, 1, pbuf[1]);
+                for (int u = nlive + 1; u < ntiles; u += kRing) {
+                    sync_issue(u, std::integral_constant<int, (J + 2) % kRing>{});
+                    if (u + 1 >= ntiles) break;
+                    sync_issue(u + 1, std::integral_constant<int, (J + 3) % kRing>{});
+                    if (u + 2 >= ntiles) break;
+                    sync_issue(u + 2, std::integral_constant<int, J>{});
+                    if (u + 3 >= ntiles) break;
+                    sync_issue(u + 3, std::integral_constant<int, (J + 1) % kRing>{});
+                }
+                vmcnt_wait<0>();
+                ring_barrier();
+            } else {
+                vmcnt_wait<0>();  // every DMA landed (none may outlive the block)
+                ring_barrier();
+                gemm1(phase_c, 1, pbuf[1]);
+            }
+        };
+        switch (rem) {
+            case 0: finish(P0{}); break;
+            case 1: finish(P1{}); break;
+            case 2: finish(P2{}); break;
+            default: finish(P3{}); break;
+        }
+    }
+    const auto ro = make_rsrc(obase, obytes);
+    lds_char* const stage = wave == 0 ? ring.k[0] : wave == 1 ? ring.k[1] : wave == 2 ? ring.k[2] : ring.k[3];
+#pragma unroll
+    for (int qb = 0; qb < 2; ++qb) {
+        const float l_tot = wave_sum_halves(l_part[qb]);
+        const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
+        lds_char* const tb = stage + qb * kRowsPerWave * kRowBytes;
+#pragma unroll
+        for (int db = 0; db < 2; ++db)
+#pragma unroll
+            for (int g4 = 0; g4 < 4; ++g4) {
+                bf16x2 x0, x1;
+                x0[0] = (__bf16)(oacc[qb][db][4 * g4 + 0] * inv);
+                x0[1] = (__bf16)(oacc[qb][db][4 * g4 + 1] * inv);
+                x1[0] = (__bf16)(oacc[qb][db][4 * g4 + 2] * inv);
+                x1[1] = (__bf16)(oacc[qb][db][4 * g4 + 3] * inv);
+                const int c = 4 * db + g4;
+                *(lds_i32x2*)(tb + l32 * kRowBytes + ((c ^ ((l32 >> 1) & 7)) << 4) + 8 * (hi ^ (l32 & 1))) =
+                    i32x2{__builtin_bit_cast(int, x0), __builtin_bit_cast(int, x1)};
+            }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int i = 0; i < kRowsPerWave / 8; ++i) {
+            const int r = 8 * i + (lane >> 3), pc = lane & 7;
+            const i32x4 raw = *(const lds_i32x4*)(tb + r * kRowBytes + (pc << 4));
+            const i32x4 v = (r & 1) ? i32x4{raw[2], raw[3], raw[0], raw[1]} : raw;
+            const int c = pc ^ ((r >> 1) & 7);
+            __builtin_amdgcn_raw_buffer_store_b128(v, ro, (wrow0 + 32 * qb + r) * p.stride_o * 2 + c * 16, 0, kStoreStream);
+        }
+        const int row = wrow0 + 32 * qb + l32;
+        if (p.lse != nullptr && hi == 0 && row < sq)
+            p.lse[(int64_t)b * p.nhead_q * sq + (int64_t)h * sq + row] =
+                (__builtin_log2f(l_tot) + m_ref[qb]) * 0.69314718055994530942f;
+    }
+}
+
 }  // namespace fmha_gfx950
 
 using namespace fmha_gfx950;
@@ -1959,6 +2317,23 @@ __global__ __launch_bounds__(FMHA_KBLOCK) void fmha_fwd_d64_bf16_chunk_balanced_
 }
 __global__ __launch_bounds__(FMHA_KBLOCK) void fmha_fwd_d64_bf16_chunk_balanced_merge_msk1(FmhaChunkArgs args) {
     chunk_merge<true>(args);
+}
+
+// ---- wide entries (this build's own; no counterpart in the reference): dense,
+// grid (nhead_q, ceil(seqlen_q / 256), batch), kBlockSize threads; causal:
+// heaviest blocks first, and the tile-major order (grid (nhead_q, batch,
+// blocks)). ----
+FMHA_ENTRY_ATTRS void fmha_fwd_d64_bf16_wide_msk0(FmhaFwdParams params) {
+    FMHA_RING(ring, kTileBytes)
+    fwd_wide<false>(params, blockIdx.z, blockIdx.x, blockIdx.y, ring);
+}
+FMHA_ENTRY_ATTRS void fmha_fwd_d64_bf16_wide_msk1(FmhaFwdParams params) {
+    FMHA_RING(ring, kTileBytes)
+    fwd_wide<true>(params, blockIdx.z, blockIdx.x, gridDim.y - 1 - blockIdx.y, ring);
+}
+FMHA_ENTRY_ATTRS void fmha_fwd_d64_bf16_wide_msk1_tilemajor(FmhaFwdParams params) {
+    FMHA_RING(ring, kTileBytes)
+    fwd_wide<true>(params, blockIdx.y, blockIdx.x, gridDim.z - 1 - blockIdx.z, ring);
 }
 
 // ---- short entries (this build's own; no counterpart in the reference):

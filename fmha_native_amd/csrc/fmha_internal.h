@@ -87,3 +87,8 @@ __global__ void fmha_fwd_d64_bf16_decode_merge_msk1_varlen(FmhaDecodeArgs args);
 // point on the static array splits no decode launch: calls on several streams
 // that needed no scratch must not start to share it).
 int64_t fmha_balanced_workspace_size(const FmhaFwdParams* p, int batch, int causal, int variant);
+
+// Wide form (see fmha_fwd_kernel.hip): 64 query rows per wave.
+__global__ void fmha_fwd_d64_bf16_wide_msk0(FmhaFwdParams params);
+__global__ void fmha_fwd_d64_bf16_wide_msk1(FmhaFwdParams params);
+__global__ void fmha_fwd_d64_bf16_wide_msk1_tilemajor(FmhaFwdParams params);
