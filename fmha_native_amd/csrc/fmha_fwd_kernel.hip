@@ -1661,29 +1661,33 @@ __device__ __forceinline__ bool sequence_item(const FmhaFwdParams& p, int rank, 
 // tile (half the DMA).  To fit 256 registers the pipeline steps by 32 keys:
 // step (t, half) issues GEMM1 of the step before, GEMM0 of the step after (8
 // MFMAs each) and the softmax of its own 32 x 64 scores, so its live state is
-// O^T 64 + Q 32 + scores 64 + P 32 registers (230 in all); the ring still moves
-// 64-key tiles, one barrier each, K(t+3) and V(t+2) in flight.
+// O^T 64 + Q 32 + scores 64 + P 32 registers (256 in all); the ring still moves
+// 64-key tiles, one barrier each, K(t+3) and V(t+2) in flight.  Frame, sums and
+// products are taken in fwd_mtile's order, so the results are its bits unless a
+// row's max outgrows its first tile's by ~11 (log2 units), where the two re-frame
+// at different keys.
 // Measured against the form it replaces: B4 H16 S2048 71.2 -> 65.2 us (1,054
 // TFLOP/s), B8 H16 S1024 38.6 -> 35.2, B16 H16 S512 23.1 -> 20.8, H16 S8192 266
 // -> 246, B32 H32 S700 174 -> 151, causal H32 S8192 283 -> 262.
 // ===========================================================================
 constexpr int kWideValuPerSlot = 5;  // 7: 3 % slower, 3: 1 %
-constexpr int kWideDsAhead = 4;      // operand reads run this many MFMAs ahead (two per read); 2: within 1 %
+constexpr int kWideDsAhead = 2;      // operand reads run this many MFMAs ahead (two per read); 4 spills
 // Slots of one step: {1 MFMA, the reads of the MFMA kWideDsAhead later, VALU};
 // MFMAs 0-7 are GEMM1's (two tr_b16 reads per two MFMAs), 8-15 GEMM0's (one b128
 // read per two).
 struct WideSchedule {
     static constexpr int reads(int m) { return m >= 16 || (m & 1) ? 0 : m < 8 ? 2 : 1; }
+    // the first step of a block has no GEMM1: MFMAs 8-15, twice the VALU each
     template <int I, bool kG1>
     static __device__ __forceinline__ void slot() {
-        constexpr int kFirst = kG1 ? 0 : 8;
+        constexpr int kRead = I + (kG1 ? 0 : 8) + kWideDsAhead;
         __builtin_amdgcn_sched_group_barrier(kSchedMFMA, 1, 0);
-        if constexpr (reads(I + kFirst + kWideDsAhead) > 0)
-            __builtin_amdgcn_sched_group_barrier(kSchedDSRead, reads(I + kFirst + kWideDsAhead), 0);
+        if constexpr (reads(kRead) > 0) __builtin_amdgcn_sched_group_barrier(kSchedDSRead, reads(kRead), 0);
         __builtin_amdgcn_sched_group_barrier(kSchedVALU, kG1 ? kWideValuPerSlot : 2 * kWideValuPerSlot, 0);
     }
     template <bool kG1, int... Is>
     static __device__ __forceinline__ void run(std::integer_sequence<int, Is...>) {
+        // the reads of the first kWideDsAhead MFMAs
         __builtin_amdgcn_sched_group_barrier(kSchedDSRead, (kG1 ? 2 : 1) * (kWideDsAhead / 2), 0);
         (slot<Is, kG1>(), ...);
     }
@@ -1754,7 +1758,8 @@ __device__ __forceinline__ void fwd_wide(const FmhaFwdParams& p, int b, int h, i
     }
     const float scale = p.scale;
     const float scale_v = in_vgpr(scale);
-    float m_ref[2] = {kMaxSeed, kMaxSeed}, l_part[2] = {0.0f, 0.0f}, l_tile[2];
+    float m_ref[2] = {kMaxSeed, kMaxSeed}, l_part[2] = {0.0f, 0.0f};
+    float l_tile[2], l_half[2];  // this step's sums of P; the tile's first half's
     f32x16 oacc[2][2];  // [qb][db]
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb)
@@ -1829,7 +1834,9 @@ __device__ __forceinline__ void fwd_wide(const FmhaFwdParams& p, int b, int h, i
         exp_half(s, pp);
         asm volatile("" ::"v"(pp[0]), "v"(pp[1]), "v"(pp[2]), "v"(pp[3]), "v"(l_tile[0]), "v"(l_tile[1]));
     };
-    auto settle = [&](const f32x16* s, bf16x8* pp) {
+    // The halves' sums meet before they join l_part: the same additions, in the
+    // same order, as a 64-key tile's of fwd_mtile.
+    auto settle = [&](int half, const f32x16* s, bf16x8* pp) {
         // as fwd_mtile's settle(), over both query blocks (the sums are >= 0)
         if (__builtin_amdgcn_ballot_w64(!(l_tile[0] + l_tile[1] <= kGrowSum))) {
             asm volatile("" ::: "memory");  // keeps the rare path a branch
@@ -1843,11 +1850,17 @@ __device__ __forceinline__ void fwd_wide(const FmhaFwdParams& p, int b, int h, i
 #pragma unroll
                     for (int r = 0; r < 16; ++r) oacc[qb][db][r] *= alpha;
                 l_part[qb] *= alpha;
+                if (half == 1) l_half[qb] *= alpha;
             }
             exp_half(s, pp);
         }
-        l_part[0] += l_tile[0];
-        l_part[1] += l_tile[1];
+#pragma unroll
+        for (int qb = 0; qb < 2; ++qb) {
+            if (half == 0)
+                l_half[qb] = l_tile[qb];
+            else
+                l_part[qb] += l_half[qb] + l_tile[qb];
+        }
     };
     f32x16 sacc[2][2];
     bf16x8 pbuf[2][4];
@@ -1871,14 +1884,14 @@ __device__ __forceinline__ void fwd_wide(const FmhaFwdParams& p, int b, int h, i
         gemm0(std::integral_constant<int, J>{}, 1, sacc[1]);
         softmax(sacc[0], pbuf[0]);
         WideSchedule::apply<!kFirst>();
-        settle(sacc[0], pbuf[0]);
+        settle(0, sacc[0], pbuf[0]);
         __builtin_amdgcn_sched_barrier(0);
         mask_half(t, 1, sacc[1]);
         gemm1(std::integral_constant<int, J>{}, 0, pbuf[0]);
         gemm0(std::integral_constant<int, (J + 1) % kRing>{}, 0, sacc[0]);
         softmax(sacc[1], pbuf[1]);
         WideSchedule::apply<true>();
-        settle(sacc[1], pbuf[1]);
+        settle(1, sacc[1], pbuf[1]);
     };
     int nlive = ntiles;
     if constexpr (kCausal) {
@@ -1925,10 +1938,19 @@ __device__ __forceinline__ void fwd_wide(const FmhaFwdParams& p, int b, int h, i
         ring_barrier();
         asm volatile("" ::"v"(qop[0][0]), "v"(qop[0][1]), "v"(qop[0][2]), "v"(qop[0][3]), "v"(qop[1][0]),
                      "v"(qop[1][1]), "v"(qop[1][2]), "v"(qop[1][3]));
+        // the first tile's exact row max, as fwd_mtile's; the second half's
+        // scores are dropped again and recomputed beside the first half's softmax
+        // (held, they spill)
+        gemm0(P0{}, 1, sacc[1]);
+        mask_half(0, 1, sacc[1]);
+        m_ref[0] = half_max(sacc[1][0]);
+        m_ref[1] = half_max(sacc[1][1]);
+        asm volatile("" : "+v"(m_ref[0]), "+v"(m_ref[1])::"memory");
         gemm0(P0{}, 0, sacc[0]);
         mask_half(0, 0, sacc[0]);
-        m_ref[0] = fmaxf(kMaxSeed, half_max(sacc[0][0]) * scale);
-        m_ref[1] = fmaxf(kMaxSeed, half_max(sacc[0][1]) * scale);
+#pragma unroll
+        for (int qb = 0; qb < 2; ++qb)
+            m_ref[qb] = fmaxf(kMaxSeed, fmaxf(half_max(sacc[0][qb]), m_ref[qb]) * scale);
         tile(0, P0{}, std::true_type{});
         int t = 1;
         for (; t + kRing <= nlive; t += kRing) {

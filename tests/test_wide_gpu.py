@@ -36,6 +36,8 @@ def test_wide_matches_regular_and_float64(b, h, hk, sq, sk, causal, rising):
     o_r, lse_r = _run(q, k, v, causal, fmha.VARIANT_REGULAR)
     d = (o.float() - o_r.float()).abs()
     assert not bool((d > 1e-2 + 1e-2 * o_r.float().abs()).any()), float(d.max())
+    if not rising:  # no row re-frames: the same operations in the same order
+        assert torch.equal(o, o_r) and torch.equal(lse, lse_r)
     # LSE: fp32 sums of the same weights in another order, on values up to |LSE|
     assert not bool(((lse - lse_r).abs() > 1e-4 + 1e-6 * lse_r.abs()).any())
     for i, j in ((0, 0), (b - 1, h - 1)):
