@@ -148,6 +148,11 @@ hipError_t fmha_fwd_d64_bf16(const FmhaFwdParams* params, int batch, int causal,
  *                         taking every CU-count-th pair; causal: one block
  *                         per pair of the first half of each (batch, head),
  *                         taking that pair's mirror next
+ * The wide form (64 query rows per wave, blocks of 256 rows) has no code of its
+ * own either: AUTO launches of dense layouts without an order flag that would run
+ * the regular or the pair form take it where its blocks are estimated to fill the
+ * compute units better (causal squares: from four blocks per compute unit and
+ * 2,560 keys).
  * The decode form has no code of its own: the query heads of a KV head share
  * one pass over its keys, whose 32-key steps the waves of a block split, and
  * with a workspace (fmha_fwd_d64_bf16_ws) the blocks too; an order flag keeps
@@ -270,7 +275,7 @@ int fmha_fwd_d64_bf16_balanced_plan(const FmhaFwdParams* params, int batch, int 
  * needed).  Returns hipSuccess or hipErrorInvalidValue. */
 hipError_t fmha_fwd_d64_bf16_check(const FmhaFwdParams* params, int batch, int causal);
 
-/* The M-tile form FMHA_VARIANT_AUTO resolves to where the decode form does not
+/* The form FMHA_VARIANT_AUTO resolves to where the decode or wide form does not
  * take the launch, for these arguments on a device with
  * `compute_units` compute units (0 = the current device's count), without
  * launching (this build's own; no counterpart in the reference).  Returns
