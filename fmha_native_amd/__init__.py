@@ -381,12 +381,17 @@ def fmha_fwd(q, k, v, causal=False, return_lse=False, seqstart_q=None, seqstart_
         lse = torch.empty(q.shape[:-1], dtype=torch.float32, device=q.device)
     p = params_from_tensors(q, k, v, o, lse, seqstart_q, seqstart_k, max_seqlen_q, max_seqlen_k)
     batch = (seqstart_q.numel() - 1) if seqstart_q is not None else q.shape[0]
+    current = torch.cuda.current_stream(q.device).cuda_stream
     if stream is None:
-        stream = torch.cuda.current_stream(q.device).cuda_stream
+        stream = current
     causal = 1 if causal else 0
     need = workspace_size(p, batch, causal)
-    if need > 0:  # the balanced form: a workspace from torch's allocator, freed after this stream's work
+    if need > 0:
+        # from torch's allocator, whose blocks belong to the current stream: on
+        # another one it must not be handed out again before this launch is done
         ws = torch.empty(need, dtype=torch.uint8, device=q.device)
+        if stream != current:
+            ws.record_stream(torch.cuda.ExternalStream(stream, device=q.device))
         fmha_fwd_d64_bf16_ws(p, batch, causal, ws.data_ptr(), need, stream)
     else:
         fmha_fwd_d64_bf16(p, batch, causal, stream)

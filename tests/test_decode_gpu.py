@@ -172,3 +172,27 @@ def test_decode_split_replays_in_a_graph():
         torch.cuda.synchronize()
         assert torch.equal(got[0], o) and torch.equal(got[1], lse)
         assert math.isfinite(float(lse.sum()))
+
+
+@pytest.mark.gpu
+def test_workspace_outlives_the_call_on_another_stream(monkeypatch):
+    """fmha_fwd on a stream that is not torch's current one: its workspace is
+    not handed out again while that stream still has work.  The launch is
+    replaced by a recorder, so nothing is written either way."""
+    q = torch.zeros(2, 16, 1, 64, device="cuda", dtype=torch.bfloat16)
+    k = torch.zeros(2, 4, 9000, 64, device="cuda", dtype=torch.bfloat16)
+    need = fmha.workspace_size(fmha.params_from_tensors(q, k, k, torch.empty_like(q)), 2, 1)
+    assert need > 0
+    seen = []
+    monkeypatch.setattr(fmha, "fmha_fwd_d64_bf16_ws", lambda p, b, c, ws, n, stream: seen.append((ws, n, stream)))
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(200_000_000)  # ~0.1 s of bounded work
+    fmha.fmha_fwd(q, k, k, causal=True, stream=side.cuda_stream)
+    busy = not side.query()
+    again = torch.empty(need, dtype=torch.uint8, device="cuda")
+    (ptr, size, stream), = seen
+    assert busy and (size, stream) == (need, side.cuda_stream)
+    assert again.data_ptr() != ptr
+    torch.cuda.synchronize()
