@@ -202,6 +202,8 @@ def time_problem(prob, steps, warmup, torch, mult=1.0, variant=0):
     form = ("balanced pair" if picked == fmha.VARIANT_BALANCED_PAIR else "balanced") + plain + \
         " (two launches: items, then the merge of split M-tiles)" if need > 0 else \
         {v: k for k, v in fmha.VARIANTS.items()}.get(picked, "?")
+    if not variant and need <= 0 and not prob.varlen:  # the launcher's own refinement of the M-tile rule has no code
+        form += " (or the wide or decode form, where the launcher estimates it faster)"
     return {"ms": ms, "wall_ms": wall * 1e3 / steps, "tflops": prob.flops() / (ms * 1e-3) / 1e12, "ramp": ramp,
             "ref_ms": ref_ms, "ref_tflops": prob.flops() / (ref_ms * 1e-3) / 1e12, "host": host, "form": form,
             "workspace_bytes": need}

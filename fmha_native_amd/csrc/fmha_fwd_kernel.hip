@@ -1666,9 +1666,9 @@ __device__ __forceinline__ bool sequence_item(const FmhaFwdParams& p, int rank, 
 // products are taken in fwd_mtile's order, so the results are its bits unless a
 // row's max outgrows its first tile's by ~11 (log2 units), where the two re-frame
 // at different keys.
-// Measured against the form it replaces: B4 H16 S2048 71.2 -> 65.2 us (1,054
-// TFLOP/s), B8 H16 S1024 38.6 -> 35.2, B16 H16 S512 23.1 -> 20.8, H16 S8192 266
-// -> 246, B32 H32 S700 174 -> 151, causal H32 S8192 283 -> 262.
+// Measured against the form it replaces: B4 H16 S2048 69.6 -> 65.0 us (1,057
+// TFLOP/s), B8 H16 S1024 37.7 -> 34.4, B16 H16 S512 22.1 -> 20.1, H16 S8192 259
+// -> 242, B32 H32 S700 162 -> 143, causal H32 S8192 272 -> 258.
 // ===========================================================================
 constexpr int kWideValuPerSlot = 5;  // 7: 3 % slower, 3: 1 %
 constexpr int kWideDsAhead = 2;      // operand reads run this many MFMAs ahead (two per read); 4 spills
