@@ -30,11 +30,12 @@ def _check(o, lse, ref_o, ref_l, tag):
     # bf16 rounding of P and O: the benchmark rule 1e-2 + 1e-2|O| (half an ulp of
     # each is 2^-9 relative; |V| rows average out); LSE is fp32 throughout
     o, lse = o.double().cpu(), lse.double().cpu()
-    bad = (o - ref_o).abs() > 1e-2 + 1e-2 * ref_o.abs()
+    # written so that NaN, the outputs' poison, is a miss
+    bad = ~((o - ref_o).abs() <= 1e-2 + 1e-2 * ref_o.abs())
     assert not bool(bad.any()), (tag, int(bad.sum()), float((o - ref_o).abs().max()))
     fin = ref_l != -INF
     assert bool((lse[~fin] == -INF).all()), tag
-    assert not bool(((lse - ref_l).abs()[fin] > 1e-3).any()), tag
+    assert bool(((lse - ref_l).abs()[fin] <= 1e-3).all()), tag
 
 
 def _params(h, hk, sq, sk):
@@ -45,6 +46,18 @@ def _params(h, hk, sq, sk):
         for f in ("stride", "nhead_stride", "batch_stride"):
             setattr(p, f"{f}_{n}", 64)
     return p
+
+
+def test_check_misses_nan():
+    """Outputs start as NaN: one left unwritten fails the comparison."""
+    ref = torch.ones(2, 64, dtype=torch.float64)
+    ok, nan = torch.ones(2, 64), torch.ones(2, 64)
+    nan[1, 3] = float("nan")
+    _check(ok, torch.ones(2), ref, torch.ones(2, dtype=torch.float64), "written")
+    with pytest.raises(AssertionError):
+        _check(nan, torch.ones(2), ref, torch.ones(2, dtype=torch.float64), "O")
+    with pytest.raises(AssertionError):
+        _check(ok, nan[:, 3], ref, torch.ones(2, dtype=torch.float64), "LSE")
 
 
 @pytest.mark.parametrize("h,hk,sq,sk,batch,chunks", [

@@ -37,4 +37,4 @@ def test_dead_waves_change_no_row(form, causal):
             assert torch.equal(outs[0][:, :, :n], outs[1][:, :, :n]), n
         else:
             d = (outs[0][:, :, :n].float() - outs[1][:, :, :n].float()).abs()
-            assert not bool((d > 1e-2 + 1e-2 * outs[1][:, :, :n].float().abs()).any()), n
+            assert bool((d <= 1e-2 + 1e-2 * outs[1][:, :, :n].float().abs()).all()), n  # NaN misses

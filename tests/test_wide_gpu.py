@@ -35,11 +35,11 @@ def test_wide_matches_regular_and_float64(b, h, hk, sq, sk, causal, rising):
     o, lse = _run(q, k, v, causal, fmha.VARIANT_AUTO)
     o_r, lse_r = _run(q, k, v, causal, fmha.VARIANT_REGULAR)
     d = (o.float() - o_r.float()).abs()
-    assert not bool((d > 1e-2 + 1e-2 * o_r.float().abs()).any()), float(d.max())
+    assert bool((d <= 1e-2 + 1e-2 * o_r.float().abs()).all()), float(d.max())  # NaN misses
     if not rising:  # no row re-frames: the same operations in the same order
         assert torch.equal(o, o_r) and torch.equal(lse, lse_r)
     # LSE: fp32 sums of the same weights in another order, on values up to |LSE|
-    assert not bool(((lse - lse_r).abs() > 1e-4 + 1e-6 * lse_r.abs()).any())
+    assert bool(((lse - lse_r).abs() <= 1e-4 + 1e-6 * lse_r.abs()).all())
     for i, j in ((0, 0), (b - 1, h - 1)):
         kv = j // (h // hk)
         ref = _f64(q[i, j:j + 1], k[i, kv:kv + 1], v[i, kv:kv + 1], causal)
