@@ -50,15 +50,15 @@ static_assert(kDecRows == 32 && FMHA_DECODE_KEY_STEP % (8 * kDecStep) == 0, "lau
 // s_waitcnt immediate for vmcnt(n) alone (gfx9 encoding)
 constexpr int wait_vmcnt(int n) { return (n & 15) | ((n >> 4) << 14) | 0x0F70; }
 
-// One (sequence, KV head, row tile): its lengths and what it sees.
+// One sequence: its lengths and packed rows.
 struct DecodeSeq {
     int64_t off_q, off_k;  // packed row offsets (varlen)
     int sq, sk;
-    int rows;    // live packed rows of the sequence
-    int kv_end;  // keys visible to the last row of the row tile
+    int rows;  // live packed rows of the sequence within the launch's bound
+    int past;  // varlen: one past the last row a grid of M-tiles would reach (>= rows)
 };
-template <bool kCausal, bool kVarlen>
-__device__ __forceinline__ DecodeSeq decode_seq(const FmhaDecodeArgs& a, int b, int row_tile) {
+template <bool kVarlen>
+__device__ __forceinline__ DecodeSeq decode_seq(const FmhaDecodeArgs& a, int b) {
     const FmhaFwdParams& p = a.p;
     DecodeSeq s;
     s.off_q = s.off_k = 0;
@@ -72,12 +72,16 @@ __device__ __forceinline__ DecodeSeq decode_seq(const FmhaDecodeArgs& a, int b, 
     }
     const int g = p.nhead_q / p.nhead_k;
     s.rows = min(s.sq, p.seqlen_q) * g;  // the launch's bound: what the workspace was sized for
-    s.kv_end = s.sk;
-    if constexpr (kCausal) {
-        const int last = (min(row_tile * kDecRows + kDecRows, s.rows) - 1) / g;  // the tile's last token
-        s.kv_end = max(0, min(s.sk, last + (s.sk - s.sq) + 1));
-    }
+    s.past = kVarlen ? min(s.sq, a.grid_rows) * g : s.rows;
     return s;
+}
+// Keys visible to the last of packed rows row0 .. end - 1 that a 32-row tile
+// from row0 holds.
+template <bool kCausal>
+__device__ __forceinline__ int visible_keys(const DecodeSeq& s, int row0, int end, int g) {
+    if constexpr (!kCausal) return s.sk;
+    const int last = (min(row0 + kDecRows, end) - 1) / g;  // the tile's last token
+    return max(0, min(s.sk, last + (s.sk - s.sq) + 1));
 }
 // Chunks with keys to walk (at least one: an empty range still has a result).
 // The last chunk takes whatever lies past the launch's seqlen_k bound.
@@ -89,26 +93,20 @@ struct DecodeLds {
     lds_char* st[kDecStages];
 };
 
+// The block's part of packed rows row0 .. end - 1 (at most 32) of KV head kvh:
+// keys k0 .. k1 - 1, into O and LSE or (split) chunk `chunk`'s partial.
 template <bool kCausal, bool kVarlen, int kDecWaves>
-__device__ __forceinline__ void fwd_decode(const FmhaDecodeArgs& a, const DecodeLds& lds) {
+__device__ __forceinline__ void decode_tile(const FmhaDecodeArgs& a, const DecodeLds& lds, const DecodeSeq& sq, int b,
+                                            int kvh, int chunk, int row0, int end, int k0, int k1, bool split) {
     const FmhaFwdParams& p = a.p;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l32 = lane & 31, hi = lane >> 5;
-    const int kvh = blockIdx.x % p.nhead_k, chunk = blockIdx.x / p.nhead_k;
-    const int row_tile = blockIdx.y, b = blockIdx.z;
-    const DecodeSeq sq = decode_seq<kCausal, kVarlen>(a, b, row_tile);
-    const int row0 = row_tile * kDecRows;
-    if (row0 >= sq.rows) return;
-    const int nlive = live_chunks(a, sq.kv_end);
-    if (chunk >= nlive) return;  // the merge skips it too
-    const int k0 = chunk * a.chunk_keys;
-    const int k1 = chunk == a.n_chunks - 1 ? sq.kv_end : min(sq.kv_end, k0 + a.chunk_keys);
     const int g = p.nhead_q / p.nhead_k;
 
     // this lane's packed row: token qi of head kvh * g + gi
     const int row = row0 + l32;
-    const bool live = row < sq.rows;
+    const bool live = row < end;
     const int qi = live ? row / g : 0, gi = live ? row - qi * g : 0;
     const int64_t head = (int64_t)kvh * g + gi;
     bf16x8 qop[4];
@@ -116,7 +114,7 @@ __device__ __forceinline__ void fwd_decode(const FmhaDecodeArgs& a, const Decode
         const __bf16* q = (const __bf16*)p.q + (kVarlen ? 0 : (int64_t)b * p.batch_stride_q) +
                           head * p.nhead_stride_q + (sq.off_q + qi) * p.stride_q + 8 * hi;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) qop[t] = *(const bf16x8*)(q + 16 * t);  // a dead row repeats row 0, unused
+        for (int t = 0; t < 4; ++t) qop[t] = *(const bf16x8*)(q + 16 * t);  // a dead row repeats the first, unused
     }
 
     const char* kbase = (const char*)((const __bf16*)p.k + (kVarlen ? 0 : (int64_t)b * p.batch_stride_k) +
@@ -274,7 +272,7 @@ __device__ __forceinline__ void fwd_decode(const FmhaDecodeArgs& a, const Decode
     l = wave_sum_halves(l);
     if (!live) return;
     // element e = 16 db + r of the lane is column 32 db + 8 (r / 4) + 4 h + r % 4
-    if (a.n_chunks > 1) {
+    if (split) {
         const int64_t slot = ((int64_t)b * p.nhead_k + kvh) * a.n_chunks + chunk;
         const int64_t at = slot * a.rows + row;
 #pragma unroll
@@ -307,6 +305,44 @@ __device__ __forceinline__ void fwd_decode(const FmhaDecodeArgs& a, const Decode
     }
 }
 
+template <bool kCausal, bool kVarlen, int kDecWaves>
+__device__ __forceinline__ void fwd_decode(const FmhaDecodeArgs& a, const DecodeLds& lds) {
+    const int nhead_k = a.p.nhead_k, g = a.p.nhead_q / nhead_k;
+    const int kvh = blockIdx.x % nhead_k, chunk = blockIdx.x / nhead_k;
+    const int b = blockIdx.z;
+    const DecodeSeq sq = decode_seq<kVarlen>(a, b);
+    int row0 = blockIdx.y * kDecRows, end = sq.rows;
+    int kv_end = 0, k0 = 0, k1 = 0;
+    bool split = a.n_chunks > 1, work = row0 < end;
+    if (work) {
+        kv_end = visible_keys<kCausal>(sq, row0, end, g);
+        work = chunk < live_chunks(a, kv_end);  // the merge skips the others too
+        k0 = chunk * a.chunk_keys;
+        k1 = chunk == a.n_chunks - 1 ? kv_end : min(kv_end, k0 + a.chunk_keys);
+    }
+    if constexpr (!kVarlen) {
+        if (work) decode_tile<kCausal, kVarlen, kDecWaves>(a, lds, sq, b, kvh, chunk, row0, end, k0, k1, split);
+    } else {
+        // A sequence with more queries than the launch's bound: the rows up to
+        // the M-tile grid's, which the forms without packed rows compute, run
+        // whole, one tile after the other, on its first block.
+        const bool tail = blockIdx.x < nhead_k && blockIdx.y == 0;
+        int next = end;
+        for (;;) {
+            if (work) decode_tile<kCausal, kVarlen, kDecWaves>(a, lds, sq, b, kvh, chunk, row0, end, k0, k1, split);
+            if (!tail || next >= sq.past) return;
+            __syncthreads();  // the exchange area becomes the ring again
+            row0 = next;
+            end = sq.past;
+            next += kDecRows;
+            k0 = 0;
+            k1 = visible_keys<kCausal>(sq, row0, end, g);
+            split = false;
+            work = true;
+        }
+    }
+}
+
 // Merge of a row's chunk partials: one wave per packed row.  Lane c holds
 // chunk c's max and sum (n_chunks <= 64), 16 lanes x 4 floats cover a partial
 // O row, so a wave reads four chunks' rows per load.
@@ -316,9 +352,10 @@ __device__ __forceinline__ void decode_merge(const FmhaDecodeArgs& a) {
     const int lane = threadIdx.x & 63;
     const int row = blockIdx.x * FMHA_DECODE_MERGE_ROWS + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kvh = blockIdx.y, b = blockIdx.z;
-    const DecodeSeq sq = decode_seq<kCausal, kVarlen>(a, b, row / kDecRows);
+    const DecodeSeq sq = decode_seq<kVarlen>(a, b);
     if (row >= sq.rows) return;
-    const int n = live_chunks(a, sq.kv_end);
+    const int g = p.nhead_q / p.nhead_k;
+    const int n = live_chunks(a, visible_keys<kCausal>(sq, row / kDecRows * kDecRows, sq.rows, g));
     const int64_t first = ((int64_t)b * p.nhead_k + kvh) * a.n_chunks;
     float m = kMaxSeed, l = 0.0f;
     if (lane < n) {
@@ -354,7 +391,6 @@ __device__ __forceinline__ void decode_merge(const FmhaDecodeArgs& a) {
     }
     if (lane >= 16) return;
     const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
-    const int g = p.nhead_q / p.nhead_k;
     const int qi = row / g, gi = row - qi * g;
     const int64_t head = (int64_t)kvh * g + gi;
     bf16x2 x0, x1;

@@ -512,7 +512,7 @@ int64_t decode_items(const FmhaFwdParams* p, int batch) {
 }
 // Fills `a` but its workspace pointers for at most `chunks` key chunks per
 // (sequence, KV head), whole steps each; returns the workspace bytes.
-int64_t decode_plan(const FmhaFwdParams* p, int batch, int chunks, int64_t cus, FmhaDecodeArgs* a) {
+int64_t decode_plan(const FmhaFwdParams* p, int batch, int causal, int chunks, int64_t cus, FmhaDecodeArgs* a) {
     const int steps = std::max(1, (p->seqlen_k + FMHA_DECODE_KEY_STEP - 1) / FMHA_DECODE_KEY_STEP);
     const int per = (steps + chunks - 1) / chunks;
     a->p = *p;
@@ -520,6 +520,11 @@ int64_t decode_plan(const FmhaFwdParams* p, int batch, int chunks, int64_t cus, 
     a->chunk_keys = per * FMHA_DECODE_KEY_STEP;
     a->n_chunks = (steps + per - 1) / per;
     a->rows = (int)decode_rows(p);
+    // what the M-tile form it replaces computes: whole M-tiles, pairs of them in the pair form
+    const int m_tiles = (p->seqlen_q + kM0 - 1) / kM0;
+    a->grid_rows = kM0 * (p->seqstart_q != nullptr && pick_form(p, batch, causal, cus) == FMHA_VARIANT_PAIR
+                              ? 2 * ((m_tiles + 1) / 2)
+                              : m_tiles);
     const int64_t pairs = (int64_t)batch * p->nhead_k;
     const int64_t blocks = pairs * a->n_chunks * ((a->rows + FMHA_DECODE_ROWS - 1) / FMHA_DECODE_ROWS);
     // eight waves (one block per CU) halve a block's serial chain; short key
@@ -625,15 +630,15 @@ int64_t decode_bytes(const FmhaFwdParams* p, int batch) {
     if (batch <= 0 || p->seqlen_q <= 0 || decode_items(p, batch) > INT32_MAX) return 0;
     FmhaDecodeArgs a;
     const int64_t cus = device_cus();
-    return decode_plan(p, batch, decode_chunks(p, batch, cus), cus, &a);
+    return decode_plan(p, batch, 0, decode_chunks(p, batch, cus), cus, &a);
 }
 // The launch with as many chunks as the workspace holds: the plan's, or one.
 hipError_t decode_run(const FmhaFwdParams* p, int batch, int causal, void* workspace, int64_t workspace_bytes,
                       hipStream_t stream) {
     FmhaDecodeArgs a;
     const int64_t cus = device_cus();
-    if (decode_plan(p, batch, decode_chunks(p, batch, cus), cus, &a) > workspace_bytes)
-        decode_plan(p, batch, 1, cus, &a);
+    if (decode_plan(p, batch, causal, decode_chunks(p, batch, cus), cus, &a) > workspace_bytes)
+        decode_plan(p, batch, causal, 1, cus, &a);
     if (a.n_chunks > 1) {
         a.part = (float*)workspace;
         a.ml = a.part + (int64_t)batch * p->nhead_k * a.n_chunks * a.rows * FMHA_HEAD_DIM;

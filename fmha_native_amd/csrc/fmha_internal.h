@@ -69,6 +69,7 @@ struct FmhaDecodeArgs {
     int chunk_keys;  // keys per chunk (the last takes the rest)
     int waves;       // waves per block: 8 (decode entries) or 4 (decode4)
     int rows;        // packed rows per (sequence, KV head): nhead_q / nhead_k * seqlen_q
+    int grid_rows;   // queries per sequence the M-tile grid would reach (varlen: seqlen_q may lie below it)
 };
 __global__ void fmha_fwd_d64_bf16_decode_msk0(FmhaDecodeArgs args);
 __global__ void fmha_fwd_d64_bf16_decode_msk1(FmhaDecodeArgs args);

@@ -30,7 +30,9 @@
  *    (src/fused/pipeline.hpp:408-418).
  *  - seqstart_q/seqstart_k non-NULL select varlen ("group") mode: device int32
  *    arrays of batch+1 prefix offsets; batch strides are ignored and
- *    seqlen_q/seqlen_k are upper bounds used only for the grid.
+ *    seqlen_q/seqlen_k are upper bounds that size the grid and steer the
+ *    choice of the kernel form (each sequence's own lengths are read on the
+ *    device).
  *  - causal is bottom-right aligned: query row i attends key j iff
  *    j <= i + (seqlen_k - seqlen_q)  (per sequence in varlen mode).
  *    A query row with no visible key gets O = 0 and LSE = -inf.
@@ -156,9 +158,9 @@ hipError_t fmha_fwd_d64_bf16(const FmhaFwdParams* params, int batch, int causal,
  * The decode form has no code of its own: the query heads of a KV head share
  * one pass over its keys, whose 32-key steps the waves of a block split, and
  * with a workspace (fmha_fwd_d64_bf16_ws) the blocks too; an order flag keeps
- * the M-tile forms.  In varlen launches
- * seqlen_q must bound every sequence's queries (rows past it are not
- * computed); seqlen_k only steers the choice and the split.
+ * the M-tile forms.  In varlen launches it computes the rows the M-tile grid
+ * would reach past seqlen_q too, one 32-row tile after the other on one block
+ * per KV head; seqlen_k only steers the choice and the split.
  * All forms give the same results up to fp32 rounding order.  Causal dense
  * launches of more than one batch whose K/V per XCD, batch x ceil(nhead_k/8)
  * x seqlen_k x 256 bytes, is at most 8 MiB run the form's tile-major entry

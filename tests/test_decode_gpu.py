@@ -155,6 +155,44 @@ def test_decode_varlen_matches_float64(causal, bound):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("causal", [0, 1])
+@pytest.mark.parametrize("h,hk,lq,lk,bound", [
+    (8, 2, [1, 100, 9, 128, 0, 33], [700, 300, 4000, 128, 64, 2500], 1),   # split with a workspace
+    (16, 16, [3, 128, 40, 2], [900, 200, 1000, 1], 3),                     # no split, one head per KV head
+    (12, 4, [64, 65, 97, 11], [2000, 1030, 70, 1500], 10),                 # the bound inside a packed tile
+    (128, 128, [1, 300, 130, 200], [2048, 300, 2048, 64], 1)])             # unmasked: two M-tiles per pair block
+def test_decode_varlen_rows_past_the_query_bound(h, hk, lq, lk, bound, causal):
+    """seqlen_q sizes a varlen launch's grid: the rows past it that the grid's
+    M-tiles reach (128 per sequence, 256 where the pair form would run) are
+    computed too, and no other row is written."""
+    batch = len(lq)
+    g = torch.Generator(device="cuda").manual_seed(h + bound)
+    rnd = lambda *s: torch.randn(s, generator=g, device="cuda").to(torch.bfloat16)
+    q, k, v = rnd(h, sum(lq), 64), rnd(hk, sum(lk), 64), rnd(hk, sum(lk), 64)
+    ss = [torch.from_numpy(np.cumsum([0] + l).astype(np.int32)).cuda() for l in (lq, lk)]
+    o = torch.empty_like(q)
+    lse = torch.empty(q.shape[:-1], device="cuda")
+    p = fmha.params_from_tensors(q, k, v, o, lse, ss[0], ss[1], bound, max(lk))
+    tile = 256 if fmha.pick_variant(p, batch, causal) == fmha.VARIANT_PAIR else 128
+    assert (tile == 256) == (h == 128 and not causal)
+    need = fmha.workspace_size(p, batch, causal)
+    ws = torch.full((max(need, 256),), 0xFF, dtype=torch.uint8, device="cuda")
+    for size in sorted({0, need}):
+        o.fill_(float("nan"))
+        lse.fill_(float("nan"))
+        fmha.fmha_fwd_d64_bf16_ws(p, batch, causal, ws.data_ptr() if size else None, size,
+                                  torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        a = c = 0
+        for nq, nk in zip(lq, lk):
+            n = min(nq, tile)
+            ref_o, ref_l = _f64(q[:, a:a + nq], k[:, c:c + nk], v[:, c:c + nk], causal)
+            _check(o[:, a:a + n], lse[:, a:a + n], ref_o[:, :n], ref_l[:, :n], (size, nq, nk))
+            assert bool(torch.isnan(o[:, a + n:a + nq].float()).all()), (size, nq, nk)
+            a, c = a + nq, c + nk
+
+
+@pytest.mark.gpu
 def test_decode_split_replays_in_a_graph():
     """A captured split launch, replayed with eager work between, equals the
     eager launch on each replay's inputs."""
