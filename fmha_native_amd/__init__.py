@@ -366,12 +366,28 @@ def params_from_tensors(q, k, v, o, lse=None, seqstart_q=None, seqstart_k=None, 
     return p
 
 
+def _stream_handle(stream):
+    """The hipStream_t, as an int, of what ctypes takes for one: an int, a
+    ctypes pointer or an object with ``_as_parameter_`` (a torch stream)."""
+    stream = getattr(stream, "_as_parameter_", stream)
+    return int(getattr(stream, "value", stream) or 0)
+
+
+def _torch_stream(handle, device):
+    """torch's stream of a handle (``ExternalStream(0)`` is a new pool stream,
+    not the null one)."""
+    import torch
+
+    return torch.cuda.ExternalStream(handle, device=device) if handle else torch.cuda.default_stream(device)
+
+
 def fmha_fwd(q, k, v, causal=False, return_lse=False, seqstart_q=None, seqstart_k=None, max_seqlen_q=None,
              max_seqlen_k=None, stream=None):
     """Attention forward on torch bf16 device tensors; returns (o, lse or None).
 
     Layouts as in :func:`params_from_tensors`; ``o`` is allocated with q's
-    shape (contiguous).  Runs on ``stream`` (default: torch's current stream).
+    shape (contiguous).  Runs on ``stream`` (a hipStream_t as int or ctypes
+    pointer, or a torch stream; default: torch's current stream).
     """
     import torch
 
@@ -382,8 +398,7 @@ def fmha_fwd(q, k, v, causal=False, return_lse=False, seqstart_q=None, seqstart_
     p = params_from_tensors(q, k, v, o, lse, seqstart_q, seqstart_k, max_seqlen_q, max_seqlen_k)
     batch = (seqstart_q.numel() - 1) if seqstart_q is not None else q.shape[0]
     current = torch.cuda.current_stream(q.device).cuda_stream
-    if stream is None:
-        stream = current
+    stream = current if stream is None else _stream_handle(stream)
     causal = 1 if causal else 0
     need = workspace_size(p, batch, causal)
     if need > 0:
@@ -391,7 +406,7 @@ def fmha_fwd(q, k, v, causal=False, return_lse=False, seqstart_q=None, seqstart_
         # another one it must not be handed out again before this launch is done
         ws = torch.empty(need, dtype=torch.uint8, device=q.device)
         if stream != current:
-            ws.record_stream(torch.cuda.ExternalStream(stream, device=q.device))
+            ws.record_stream(_torch_stream(stream, q.device))
         fmha_fwd_d64_bf16_ws(p, batch, causal, ws.data_ptr(), need, stream)
     else:
         fmha_fwd_d64_bf16(p, batch, causal, stream)
