@@ -373,12 +373,25 @@ def _stream_handle(stream):
     return int(getattr(stream, "value", stream) or 0)
 
 
-def _torch_stream(handle, device):
-    """torch's stream of a handle (``ExternalStream(0)`` is a new pool stream,
-    not the null one)."""
+def _other_stream(stream, device):
+    """(torch's stream of ``stream``, the current one) where they differ, else
+    None: torch's allocator gives out blocks of the current stream's pool, in
+    whose order alone they are free."""
     import torch
 
-    return torch.cuda.ExternalStream(handle, device=device) if handle else torch.cuda.default_stream(device)
+    current = torch.cuda.current_stream(device)
+    handle = _stream_handle(stream)
+    if handle == current.cuda_stream:
+        return None
+    # ExternalStream(0) would be a new pool stream, not the null one
+    side = torch.cuda.ExternalStream(handle, device=device) if handle else torch.cuda.default_stream(device)
+    return side, current
+
+
+def _record(tensors, stream):
+    for t in tensors:
+        if t is not None:
+            t.record_stream(stream)
 
 
 def fmha_fwd(q, k, v, causal=False, return_lse=False, seqstart_q=None, seqstart_k=None, max_seqlen_q=None,
@@ -387,26 +400,33 @@ def fmha_fwd(q, k, v, causal=False, return_lse=False, seqstart_q=None, seqstart_
 
     Layouts as in :func:`params_from_tensors`; ``o`` is allocated with q's
     shape (contiguous).  Runs on ``stream`` (a hipStream_t as int or ctypes
-    pointer, or a torch stream; default: torch's current stream).
+    pointer, or a torch stream; default: torch's current stream).  On another
+    stream than the current one, the caller orders the inputs' writers before
+    the call and the outputs' readers after it, as for any launch there; the
+    memory of the outputs and the workspace is that stream's, and no tensor of
+    the call is reused before both streams are done with it.
     """
     import torch
 
+    other = _other_stream(stream, q.device) if stream is not None and q.is_cuda else None
+    if other is not None:
+        side, current = other
+        with torch.cuda.stream(side):
+            o, lse = fmha_fwd(q, k, v, causal, return_lse, seqstart_q, seqstart_k, max_seqlen_q, max_seqlen_k)
+        _record((q, k, v, seqstart_q, seqstart_k), side)
+        _record((o, lse), current)
+        return o, lse
     o = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     lse = None
     if return_lse:
         lse = torch.empty(q.shape[:-1], dtype=torch.float32, device=q.device)
     p = params_from_tensors(q, k, v, o, lse, seqstart_q, seqstart_k, max_seqlen_q, max_seqlen_k)
     batch = (seqstart_q.numel() - 1) if seqstart_q is not None else q.shape[0]
-    current = torch.cuda.current_stream(q.device).cuda_stream
-    stream = current if stream is None else _stream_handle(stream)
+    stream = torch.cuda.current_stream(q.device).cuda_stream
     causal = 1 if causal else 0
     need = workspace_size(p, batch, causal)
-    if need > 0:
-        # from torch's allocator, whose blocks belong to the current stream: on
-        # another one it must not be handed out again before this launch is done
+    if need > 0:  # from torch's allocator, freed after this stream's work
         ws = torch.empty(need, dtype=torch.uint8, device=q.device)
-        if stream != current:
-            ws.record_stream(_torch_stream(stream, q.device))
         fmha_fwd_d64_bf16_ws(p, batch, causal, ws.data_ptr(), need, stream)
     else:
         fmha_fwd_d64_bf16(p, batch, causal, stream)
@@ -429,8 +449,18 @@ def merge_partials(o_parts, lse_parts, o=None, lse=None, stream=None):
     ``o_parts``: bf16 [n, ..., 64] and ``lse_parts``: float32 [n, ...] with the
     same ``...`` (rows in LSE order, e.g. [B, H, S] or [H, T]), both contiguous.
     Returns (o, lse) with shapes [..., 64] and [...]; ``o``/``lse`` may be given.
+    ``stream`` as in :func:`fmha_fwd`.
     """
     import torch
+
+    other = _other_stream(stream, o_parts.device) if stream is not None and o_parts.is_cuda else None
+    if other is not None:
+        side, current = other
+        with torch.cuda.stream(side):
+            out = merge_partials(o_parts, lse_parts, o, lse)
+        _record((o_parts, lse_parts, o, lse), side)
+        _record([t for t, given in zip(out, (o, lse)) if given is None], current)
+        return out
 
     if o_parts.dtype not in (torch.bfloat16, torch.int16) or lse_parts.dtype != torch.float32:
         raise ValueError("o_parts must be bfloat16 (or int16 bf16 bits) and lse_parts float32")
@@ -452,8 +482,7 @@ def merge_partials(o_parts, lse_parts, o=None, lse=None, stream=None):
     tensors = (o_parts, lse_parts, o, lse)
     if not all(t.is_cuda for t in tensors) or len({t.device for t in tensors}) != 1:
         raise ValueError("all tensors must be on the same GPU")
-    if stream is None:
-        stream = torch.cuda.current_stream(o_parts.device).cuda_stream
+    stream = torch.cuda.current_stream(o_parts.device).cuda_stream
     fmha_merge_d64_bf16(n, rows, o_parts.data_ptr(), rows * HEAD_DIM, lse_parts.data_ptr(), rows, HEAD_DIM,
                         o.data_ptr(), lse.data_ptr(), stream)
     return o, lse
