@@ -24,7 +24,7 @@ import numpy as np
 
 __all__ = [
     "FmhaError", "FmhaFwdParams", "LIB_PATH", "load_library", "fmha_fwd_d64_bf16", "check_params",
-    "tile_config", "pick_variant", "tile_major", "fill_ref", "fill_normal", "varlen_lengths", "params_from_tensors", "fmha_fwd",
+    "tile_config", "launch_form", "pick_variant", "tile_major", "fill_ref", "fill_normal", "varlen_lengths", "params_from_tensors", "fmha_fwd",
     "fmha_merge_d64_bf16", "merge_partials", "MERGE_MAX_PARTS",
     "LOG2E", "HIP_ERROR_INVALID_VALUE", "VARIANT_AUTO", "VARIANT_REGULAR", "VARIANT_SPLITKV", "VARIANT_PAIR",
     "VARIANT_BALANCED", "VARIANT_SHORT", "VARIANT_BALANCED_PAIR", "VARIANT_PAIR_STREAM", "fmha_fwd_d64_bf16_ws", "workspace_size", "balanced_plan",
@@ -89,6 +89,8 @@ def load_library(path=LIB_PATH):
     lib.fmha_fwd_d64_bf16_check.restype = ctypes.c_int
     lib.fmha_fwd_d64_bf16_pick_variant.argtypes = [P, ctypes.c_int, ctypes.c_int, ctypes.c_int]
     lib.fmha_fwd_d64_bf16_pick_variant.restype = ctypes.c_int
+    lib.fmha_fwd_d64_bf16_form.argtypes = [P, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int64]
+    lib.fmha_fwd_d64_bf16_form.restype = ctypes.c_int
     lib.fmha_fwd_d64_bf16_tile_major.argtypes = [P, ctypes.c_int, ctypes.c_int]
     lib.fmha_fwd_d64_bf16_tile_major.restype = ctypes.c_int
     lib.fmha_fwd_d64_bf16_ws.argtypes = [P, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_int64,
@@ -134,6 +136,9 @@ VARIANT_SEQUENCE_ORDER = 64
 VARIANTS = {"auto": VARIANT_AUTO, "regular": VARIANT_REGULAR, "splitkv": VARIANT_SPLITKV, "pair": VARIANT_PAIR,
             "balanced": VARIANT_BALANCED, "short": VARIANT_SHORT,
             "balanced_pair": VARIANT_BALANCED_PAIR, "pair_stream": VARIANT_PAIR_STREAM}
+# forms without a variant code, as launch_form() reports them
+FORM_DECODE, FORM_CHUNK, FORM_WIDE = 9, 10, 11
+FORMS = {**{c: n for n, c in VARIANTS.items() if c}, FORM_DECODE: "decode", FORM_CHUNK: "chunk", FORM_WIDE: "wide"}
 ORDERS = {"reference": VARIANT_REFERENCE_ORDER, "tilemajor": VARIANT_TILE_MAJOR_ORDER,
           "sequence": VARIANT_SEQUENCE_ORDER}
 
@@ -220,11 +225,19 @@ def check_params(params, batch, causal):
     return load_library().fmha_fwd_d64_bf16_check(ctypes.byref(params), int(batch), int(causal))
 
 
+def launch_form(params, batch, causal, variant=VARIANT_AUTO, workspace_bytes=0):
+    """The form a launch with these arguments and a workspace of this size runs
+    on the current device: a VARIANT_* or FORM_* code (names in ``FORMS``), 0
+    when nothing is launched, -1 for rejected arguments.  Host only."""
+    return load_library().fmha_fwd_d64_bf16_form(ctypes.byref(params), int(batch), int(causal), int(variant),
+                                                 int(workspace_bytes))
+
+
 def pick_variant(params, batch, causal, compute_units=0):
     """The M-tile form VARIANT_AUTO resolves to on a device with
-    ``compute_units`` CUs (0 = the current device's), where the decode form
-    (few query rows, no code of its own) does not take the launch; -1 for
-    rejected arguments.  Host only."""
+    ``compute_units`` CUs (0 = the current device's), where no other form
+    takes the launch (:func:`launch_form` reports those too); -1 for rejected
+    arguments.  Host only."""
     return load_library().fmha_fwd_d64_bf16_pick_variant(ctypes.byref(params), int(batch), int(causal),
                                                           int(compute_units))
 

@@ -139,9 +139,8 @@ int pick_variant(int64_t blocks, int64_t pairs, int causal, int seqlen_k, int64_
 // of L2 before its later M-tiles run.  Measured on causal grids (regular
 // form): +19% B8 H16 S1024, +8% B4 H16 S2048, +6% B16 H8 S2048, +2-6% B2 H16
 // S4096/S8192, and -1 to -5% above 8 MiB.
-bool use_tilemajor(const FmhaFwdParams* p, int batch, int causal) {
+bool use_tilemajor(const FmhaFwdParams* p, int batch, int causal, const DeviceShape& d) {
     if (!causal || batch < 2 || p->seqstart_q != nullptr) return false;
-    const DeviceShape d = device_shape();
     // batch x heads-per-XCD x seqlen_k <= 2 x L2 / 256 B, evaluated without overflow
     const int64_t limit = 2 * (int64_t)d.l2_bytes / 256;
     const int64_t rows = (int64_t)batch * (((int64_t)p->nhead_k + d.xccs - 1) / d.xccs);  // <= 2^16 * 2^31
@@ -183,17 +182,17 @@ bool compact_applies(const FmhaFwdParams* p, int batch, int causal) {
 // +13 %, H16 -3.3 % / +2.2 %, H32 -15 % / -2.5 %; 16 lengths 100-4000 H8
 // +2.6 % / +5.1 %, H16 -12 % / -2.3 %; 32 and 64 sequences of 16-2048 tokens
 // H16 -17 to -29 % / -12 to -41 %; 16 x 512 H16 -1.1 % / -9.7 %.
-int varlen_order(const FmhaFwdParams* p, int batch, int causal, int order) {
+int varlen_order(const FmhaFwdParams* p, int batch, int causal, int order, int64_t cus) {
     if (!compact_applies(p, batch, causal) || order == kOrderReference) return kOrderReference;
     if (order != kOrderAuto) return order;
     const int64_t blocks = (int64_t)p->nhead_q * ((p->seqlen_q + kM0 - 1) / kM0) * batch;  // the grid: a bound
-    return batch <= 8 && blocks <= 16 * (int64_t)device_cus() ? kOrderSequence : kOrderReference;
+    return batch <= 8 && blocks <= 16 * cus ? kOrderSequence : kOrderReference;
 }
 // Dense causal batches on the tile-major entries?
-bool dense_tile_major(const FmhaFwdParams* p, int batch, int causal, int order) {
+bool dense_tile_major(const FmhaFwdParams* p, int batch, int causal, int order, const DeviceShape& d) {
     if (order == kOrderReference || order == kOrderSequence) return false;
     if (order == kOrderTileMajor) return causal && batch >= 2 && p->seqstart_q == nullptr;
-    return use_tilemajor(p, batch, causal);
+    return use_tilemajor(p, batch, causal, d);
 }
 
 // Keys up to which the automatic choice takes the short form: on every grid
@@ -587,21 +586,24 @@ bool decode_faster(const FmhaFwdParams* p, const DecodeAsk& a) {
         5.9 + (2 * items > a.cus ? 0.8 : 0.65) * ((steps + chunks - 1) / chunks) + (chunks > 1 ? 3.2 : 0.0);
     return us < 0.97 * mtile_us(p, a.batch, a.causal, a.cus, a.workspace != 0).us;
 }
-bool takes_decode(const FmhaFwdParams* p, int batch, int causal, int variant, bool split, bool workspace) {
-    if (variant != FMHA_VARIANT_AUTO || batch <= 0 || p->seqlen_q <= 0 || p->seqlen_k < 128) return false;
+bool takes_decode(const FmhaFwdParams* p, int batch, int causal, int64_t cus, bool split, bool workspace) {
+    if (p->seqlen_k < 128) return false;
     if (decode_rows(p) <= 128 && (p->seqlen_q <= 32 || (p->seqlen_q <= 64 && p->seqlen_k >= 1024))) return true;
     if (p->seqstart_q != nullptr) return false;
-    // the estimates walk the M-tiles: a thread's last answer is kept (it
-    // depends on the shape only)
-    thread_local DecodeAsk last{-1, -1, -1, -1, -1, -1, -1, -1, -1};
-    thread_local bool last_answer = false;
-    const DecodeAsk ask{p->seqlen_q, p->seqlen_k, p->nhead_q, p->nhead_k, batch, causal,
-                        split, workspace, device_cus()};
-    if (!(ask == last)) {
-        last_answer = decode_faster(p, ask);
-        last = ask;
+    // the estimates walk the M-tiles: a thread's last answers with and without
+    // a workspace are kept (they depend on the shape only)
+    struct Kept {
+        DecodeAsk ask{-1, -1, -1, -1, -1, -1, -1, -1, -1};
+        bool answer = false;
+    };
+    thread_local Kept kept[2];
+    Kept& last = kept[workspace ? 1 : 0];
+    const DecodeAsk ask{p->seqlen_q, p->seqlen_k, p->nhead_q, p->nhead_k, batch, causal, split, workspace, cus};
+    if (!(ask == last.ask)) {
+        last.answer = decode_faster(p, ask);
+        last.ask = ask;
     }
-    return last_answer;
+    return last.answer;
 }
 
 hipError_t decode_launch(const FmhaDecodeArgs& a, int batch, int causal, hipStream_t stream) {
@@ -626,17 +628,15 @@ hipError_t decode_launch(const FmhaDecodeArgs& a, int batch, int causal, hipStre
     return hipGetLastError();
 }
 // Workspace bytes of the split launch (0: never split).
-int64_t decode_bytes(const FmhaFwdParams* p, int batch) {
-    if (batch <= 0 || p->seqlen_q <= 0 || decode_items(p, batch) > INT32_MAX) return 0;
+int64_t decode_bytes(const FmhaFwdParams* p, int batch, int64_t cus) {
+    if (decode_items(p, batch) > INT32_MAX) return 0;
     FmhaDecodeArgs a;
-    const int64_t cus = device_cus();
     return decode_plan(p, batch, 0, decode_chunks(p, batch, cus), cus, &a);
 }
 // The launch with as many chunks as the workspace holds: the plan's, or one.
-hipError_t decode_run(const FmhaFwdParams* p, int batch, int causal, void* workspace, int64_t workspace_bytes,
-                      hipStream_t stream) {
+hipError_t decode_run(const FmhaFwdParams* p, int batch, int causal, int64_t cus, void* workspace,
+                      int64_t workspace_bytes, hipStream_t stream) {
     FmhaDecodeArgs a;
-    const int64_t cus = device_cus();
     if (decode_plan(p, batch, causal, decode_chunks(p, batch, cus), cus, &a) > workspace_bytes)
         decode_plan(p, batch, causal, 1, cus, &a);
     if (a.n_chunks > 1) {
@@ -670,12 +670,11 @@ bool chunk_plan_build(const FmhaFwdParams* p, int batch, int causal, int64_t cus
     *bytes = (int64_t)batch * p->nhead_q * slots * FMHA_BALANCED_PART_BYTES;
     return true;
 }
-// The plan of a launch with this variant (the automatic choice without an
-// order flag); fills `a` but its workspace pointer.  It depends on the shape
-// only, so the last one built on a thread is kept, as the balanced form's.
-bool chunk_plan(const FmhaFwdParams* p, int batch, int causal, int variant, FmhaChunkArgs* a, int64_t* bytes) {
-    if (variant != FMHA_VARIANT_AUTO || batch <= 0 || p->seqlen_q <= 0 || p->seqstart_q != nullptr) return false;
-    const int64_t cus = device_cus();
+// The plan of an automatic launch without an order flag; fills `a` but its
+// workspace pointer.  It depends on the shape only, so the last one built on a
+// thread is kept, as the balanced form's.
+bool chunk_plan(const FmhaFwdParams* p, int batch, int causal, int64_t cus, FmhaChunkArgs* a, int64_t* bytes) {
+    if (p->seqstart_q != nullptr) return false;
     struct Key {
         int seqlen_q, seqlen_k, nhead_q, batch, causal;
         int64_t cus;
@@ -718,7 +717,8 @@ hipError_t chunk_launch(const FmhaChunkArgs& a, int batch, int causal, hipStream
 }
 
 // Whether the automatic choice takes the wide form (64 rows per wave, 256 per
-// block): dense layouts whose M-tile form would be the regular or the pair form.
+// block): dense layouts whose M-tile form would be the regular or the pair form
+// (`form`).
 //  * Blocks of about equal work (no mask, or a causal key range much longer
 //    than the queries): a CU with two blocks takes 1.86 us per key tile of both
 //    and one block alone 1.08 (regular 1.12 and 0.60 for half the rows, pair
@@ -733,11 +733,8 @@ hipError_t chunk_launch(const FmhaChunkArgs& a, int batch, int causal, hipStream
 //    little from 2,560 keys: H32 S8192 283 / 262, H16 S16384 543 / 501, B12 H32
 //    S3000 519 / 478, B4 H32 S4096 304 / 290; B16 H16 S2048 179 / 178, B16 H16
 //    S1024 56 / 63, H24 S6000 (576 blocks) 122 / 130, H16 S8192 (512) 142 / 155.
-bool takes_wide(const FmhaFwdParams* p, int batch, int causal, int variant, int64_t cus) {
-    if (variant != FMHA_VARIANT_AUTO || p->seqstart_q != nullptr || batch <= 0 || p->seqlen_q <= 0 ||
-        p->seqlen_k <= 0)
-        return false;
-    const int form = pick_form(p, batch, causal, cus);
+bool takes_wide(const FmhaFwdParams* p, int batch, int causal, int form, int64_t cus) {
+    if (p->seqstart_q != nullptr || p->seqlen_k <= 0) return false;
     if (form != FMHA_VARIANT_REGULAR && form != FMHA_VARIANT_PAIR) return false;
     const int m_tiles = (p->seqlen_q + kM0 - 1) / kM0;
     const int longest = mtile_tiles(p, causal, m_tiles - 1);
@@ -753,80 +750,90 @@ bool takes_wide(const FmhaFwdParams* p, int batch, int causal, int variant, int6
     return us(wide, 1.86, 1.08) < 0.97 * other;
 }
 
-// The plan mode of a variant that takes a workspace, or -1 for the others.
+// The plan mode of a form that runs a balanced plan (AUTO: might), or -1.
 int plan_mode(int v) {
     return v == FMHA_VARIANT_AUTO            ? kPlanAuto
            : v == FMHA_VARIANT_BALANCED      ? kPlanSingle
            : v == FMHA_VARIANT_BALANCED_PAIR ? kPlanPair
                                              : -1;
 }
+// The XCD count a balanced plan is ordered for: the reference-order flag keeps
+// the plain heaviest-first table (the results are the same bit for bit: the
+// items do not change).
+int plan_xccs(int order, const DeviceShape& d) { return order == kOrderReference ? 1 : d.xccs; }
 
-}  // namespace
-
-extern "C" int fmha_fwd_d64_bf16_balanced_plan(const FmhaFwdParams* p, int batch, int causal, int compute_units,
-                                               int xccs, int force, unsigned short* items, int capacity,
-                                               int* split_from) {
-    if (fmha_fwd_d64_bf16_check(p, batch, causal) != hipSuccess || compute_units < 0 || xccs < 0) return -1;
-    if (force < kPlanAuto || force > kPlanPair) return -1;
-    FmhaBalancedArgs a;
-    if (!balanced_plan(p, batch, causal, compute_units > 0 ? compute_units : device_cus(),
-                       xccs > 0 ? xccs : device_shape().xccs, force, &a, nullptr))
-        return 0;
-    if (items != nullptr)
-        for (int i = 0; i < a.n_items && i < capacity; ++i) items[i] = a.item[i];
-    if (split_from != nullptr) *split_from = a.split_from;
-    return a.n_items;
-}
-
-int64_t fmha_balanced_workspace_size(const FmhaFwdParams* p, int batch, int causal, int variant) {
-    if (fmha_fwd_d64_bf16_check(p, batch, causal) != hipSuccess) return -1;
-    if (order_of(variant) < 0) return -1;
-    const int mode = plan_mode(variant & ~kOrderFlags);
-    if (mode < 0) return 0;
-    if (takes_decode(p, batch, causal, variant, false, false)) return 0;
-    int64_t bytes = 0;
-    // the same plan (and cache entry) as the launch with this variant
-    const int xccs = order_of(variant) == kOrderReference ? 1 : device_shape().xccs;
-    if (!balanced_plan(p, batch, causal, device_cus(), xccs, mode, nullptr, &bytes)) return 0;
-    return bytes;
-}
-
-extern "C" int64_t fmha_fwd_d64_bf16_workspace_size(const FmhaFwdParams* p, int batch, int causal, int variant) {
-    const hipError_t chk = fmha_fwd_d64_bf16_check(p, batch, causal);
-    if (chk != hipSuccess) return -1;
-    int64_t bytes = 0;
-    if (takes_decode(p, batch, causal, variant, true, true)) return decode_bytes(p, batch);
-    if (chunk_plan(p, batch, causal, variant, nullptr, &bytes)) return bytes;
-    return fmha_balanced_workspace_size(p, batch, causal, variant);
-}
-
-extern "C" hipError_t fmha_fwd_d64_bf16_ws(const FmhaFwdParams* p, int batch, int causal, int variant,
-                                           void* workspace, int64_t workspace_bytes, hipStream_t stream) {
-    const hipError_t chk = fmha_fwd_d64_bf16_check(p, batch, causal);
-    if (chk != hipSuccess) return chk;
-    if (order_of(variant) < 0) return hipErrorInvalidValue;
-    const int mode = plan_mode(variant & ~kOrderFlags);
-    if (mode < 0) return fmha_fwd_d64_bf16_variant(p, batch, causal, variant, stream);
-    if (workspace_bytes < 0 || (workspace == nullptr && workspace_bytes != 0) ||
-        (reinterpret_cast<uintptr_t>(workspace) & 255u))
-        return hipErrorInvalidValue;
-    if (batch == 0 || p->seqlen_q == 0) return hipSuccess;
-    if (takes_decode(p, batch, causal, variant, decode_bytes(p, batch) <= workspace_bytes, workspace_bytes > 0))
-        return decode_run(p, batch, causal, workspace, workspace_bytes, stream);
-    FmhaChunkArgs c;
-    int64_t chunk_bytes = 0;
-    if (chunk_plan(p, batch, causal, variant, &c, &chunk_bytes) && chunk_bytes <= workspace_bytes) {
-        c.part = (float*)workspace;
-        return chunk_launch(c, batch, causal, stream);
+// A launch's parts, once: the form, the block order and the device they were
+// decided for.  The launch and fmha_fwd_d64_bf16_form() take it from here.
+struct Launch {
+    int form = -1;  // FMHA_VARIANT_* or FMHA_FORM_*; 0: nothing to launch; -1: rejected
+    int order = kOrderAuto;
+    bool plan_auto = false;  // a balanced form the automatic choice took
+    DeviceShape dev{};
+};
+// `workspace`: the call has a workspace argument (of `bytes` bytes); the forms
+// that need one are rejected without.
+Launch decide(const FmhaFwdParams* p, int batch, int causal, int variant, bool workspace, int64_t bytes) {
+    Launch l;
+    l.order = order_of(variant);
+    if (l.order < 0) return l;  // more than one order flag
+    const int v = variant & ~kOrderFlags;
+    const bool varlen = p->seqstart_q != nullptr;
+    const bool empty = batch == 0 || p->seqlen_q == 0;
+    switch (v) {  // 4 is a retired value
+        case FMHA_VARIANT_PAIR_STREAM:
+            if (varlen) return l;  // dense layouts only
+            [[fallthrough]];
+        case FMHA_VARIANT_REGULAR:
+        case FMHA_VARIANT_SPLITKV:
+        case FMHA_VARIANT_PAIR:
+        case FMHA_VARIANT_SHORT:
+            l.form = empty ? 0 : v;
+            if (!empty) l.dev = device_shape();
+            return l;
+        case FMHA_VARIANT_BALANCED:
+        case FMHA_VARIANT_BALANCED_PAIR:
+            if (!workspace) return l;
+            break;
+        case FMHA_VARIANT_AUTO: break;
+        default: return l;
     }
-    FmhaBalancedArgs a;
+    if (empty) {
+        l.form = 0;
+        return l;
+    }
+    l.dev = device_shape();
+    const int64_t cus = l.dev.cus;
     int64_t need = 0;
-    // the reference-order flag keeps the plain heaviest-first table (the
-    // results are the same bit for bit: the items do not change)
-    const int xccs = order_of(variant) == kOrderReference ? 1 : device_shape().xccs;
-    const bool plan = balanced_plan(p, batch, causal, device_cus(), xccs, mode, &a, &need);
-    if (mode != kPlanAuto && (!plan || need > workspace_bytes)) return hipErrorInvalidValue;
-    if (!plan || need > workspace_bytes) return fmha_fwd_d64_bf16_variant(p, batch, causal, variant, stream);
+    if (v == FMHA_VARIANT_AUTO) {
+        if (l.order == kOrderAuto) {
+            if (takes_decode(p, batch, causal, cus, decode_bytes(p, batch, cus) <= bytes, bytes > 0)) {
+                l.form = FMHA_FORM_DECODE;
+                return l;
+            }
+            if (bytes > 0 && chunk_plan(p, batch, causal, cus, nullptr, &need) && need <= bytes) {
+                l.form = FMHA_FORM_CHUNK;
+                return l;
+            }
+        }
+        // an automatic plan always splits something, so it needs a workspace
+        l.plan_auto = bytes > 0 && balanced_plan(p, batch, causal, cus, plan_xccs(l.order, l.dev), kPlanAuto, nullptr,
+                                                 &need) && need <= bytes;
+        l.form = l.plan_auto ? FMHA_VARIANT_BALANCED : pick_form(p, batch, causal, cus);
+        if (!l.plan_auto && l.order == kOrderAuto && takes_wide(p, batch, causal, l.form, cus))
+            l.form = FMHA_FORM_WIDE;
+        return l;
+    }
+    if (balanced_plan(p, batch, causal, cus, plan_xccs(l.order, l.dev), plan_mode(v), nullptr, &need) && need <= bytes)
+        l.form = v;
+    return l;
+}
+
+hipError_t balanced_launch(const FmhaFwdParams* p, int batch, int causal, const Launch& l, void* workspace,
+                           hipStream_t stream) {
+    FmhaBalancedArgs a;
+    const int mode = l.plan_auto ? (int)kPlanAuto : plan_mode(l.form);
+    if (!balanced_plan(p, batch, causal, l.dev.cus, plan_xccs(l.order, l.dev), mode, &a, nullptr))
+        return hipErrorInvalidValue;
     a.p = *p;
     a.part = (float*)workspace;
     if (a.pair)
@@ -842,39 +849,11 @@ extern "C" hipError_t fmha_fwd_d64_bf16_ws(const FmhaFwdParams* p, int batch, in
     return hipGetLastError();
 }
 
-extern "C" int fmha_fwd_d64_bf16_pick_variant(const FmhaFwdParams* p, int batch, int causal, int compute_units) {
-    if (fmha_fwd_d64_bf16_check(p, batch, causal) != hipSuccess || compute_units < 0) return -1;
-    const int64_t cus = compute_units > 0 ? compute_units : device_cus();
-    return pick_form(p, batch, causal, cus);
-}
-
-extern "C" int fmha_fwd_d64_bf16_tile_major(const FmhaFwdParams* p, int batch, int causal) {
-    if (fmha_fwd_d64_bf16_check(p, batch, causal) != hipSuccess) return -1;
-    if (p->seqlen_q == 0 || batch == 0) return 0;  // nothing is launched
-    if (dense_tile_major(p, batch, causal, kOrderAuto)) return 1;
-    // varlen: the compact orders, which only the regular form has
-    if (pick_form(p, batch, causal, device_cus()) != FMHA_VARIANT_REGULAR) return 0;
-    const int o = varlen_order(p, batch, causal, kOrderAuto);
-    return o == kOrderTileMajor ? 1 : o == kOrderSequence ? 2 : 0;
-}
-
-extern "C" hipError_t fmha_fwd_d64_bf16_variant(const FmhaFwdParams* p, int batch, int causal, int variant,
-                                                hipStream_t stream) {
-    const hipError_t chk = fmha_fwd_d64_bf16_check(p, batch, causal);
-    if (chk != hipSuccess) return chk;
-    const int order = order_of(variant);
-    if (order < 0) return hipErrorInvalidValue;  // more than one order flag
-    const bool tile_major = dense_tile_major(p, batch, causal, order);
-    const bool decode = takes_decode(p, batch, causal, variant, false, false);
-    variant &= ~kOrderFlags;
-    // the balanced forms need fmha_fwd_d64_bf16_ws; 4 is a retired value
-    if (!(variant == FMHA_VARIANT_AUTO || variant == FMHA_VARIANT_REGULAR || variant == FMHA_VARIANT_SPLITKV ||
-          variant == FMHA_VARIANT_PAIR || variant == FMHA_VARIANT_SHORT || variant == FMHA_VARIANT_PAIR_STREAM))
-        return hipErrorInvalidValue;
+// The M-tile forms and the wide form.
+hipError_t grid_launch(const FmhaFwdParams* p, int batch, int causal, const Launch& l, hipStream_t stream) {
+    const int variant = l.form;
     const bool varlen = p->seqstart_q != nullptr;
-    if (variant == FMHA_VARIANT_PAIR_STREAM && varlen) return hipErrorInvalidValue;  // dense layouts only
-    if (batch == 0 || p->seqlen_q == 0) return hipSuccess;  // nothing to compute
-    if (decode) return decode_run(p, batch, causal, nullptr, 0, stream);
+    const bool tile_major = dense_tile_major(p, batch, causal, l.order, l.dev);
     const int m_tiles = (p->seqlen_q + kM0 - 1) / kM0;
     const dim3 grid(p->nhead_q, m_tiles, batch);
     if (variant == FMHA_VARIANT_PAIR_STREAM) {
@@ -884,7 +863,7 @@ extern "C" hipError_t fmha_fwd_d64_bf16_variant(const FmhaFwdParams* p, int batc
         const int64_t items = (int64_t)p->nhead_q * ny * batch;
         if (items >= INT32_MAX) return hipErrorInvalidValue;  // item numbers are ints
         const int64_t blocks = causal ? (int64_t)p->nhead_q * ((ny + 1) / 2) * batch
-                                      : std::min<int64_t>(items, device_cus());
+                                      : std::min<int64_t>(items, l.dev.cus);
         FmhaStreamArgs a;
         a.p = *p;
         a.ny = (int)ny;
@@ -897,7 +876,7 @@ extern "C" hipError_t fmha_fwd_d64_bf16_variant(const FmhaFwdParams* p, int batc
                                stream, a);
         return hipGetLastError();
     }
-    if (order == kOrderAuto && takes_wide(p, batch, causal, variant, device_cus())) {
+    if (variant == FMHA_FORM_WIDE) {
         const int blocks = (m_tiles + 1) / 2;
         if (tile_major)
             hipLaunchKernelGGL(fmha_fwd_d64_bf16_wide_msk1_tilemajor, dim3(p->nhead_q, batch, blocks), dim3(kBlockSize),
@@ -910,8 +889,6 @@ extern "C" hipError_t fmha_fwd_d64_bf16_variant(const FmhaFwdParams* p, int batc
                                stream, *p);
         return hipGetLastError();
     }
-    if (variant == FMHA_VARIANT_AUTO)
-        variant = pick_form(p, batch, causal, device_cus());
     if (variant == FMHA_VARIANT_SHORT) {
         using Entry = void (*)(FmhaFwdParams);
         static const Entry entries[2][2] = {{fmha_fwd_d64_bf16_short_msk0, fmha_fwd_d64_bf16_short_msk0_varlen},
@@ -965,7 +942,7 @@ extern "C" hipError_t fmha_fwd_d64_bf16_variant(const FmhaFwdParams* p, int batc
     const dim3 block(kBlockSize);
     if (varlen) {
         if (causal)
-            switch (varlen_order(p, batch, causal, order)) {
+            switch (varlen_order(p, batch, causal, l.order, l.dev.cus)) {
                 case kOrderTileMajor:
                     hipLaunchKernelGGL(fmha_fwd_d64_bf16_msk1_varlen_tilemajor, grid, block, 0, stream, *p);
                     break;
@@ -984,6 +961,108 @@ extern "C" hipError_t fmha_fwd_d64_bf16_variant(const FmhaFwdParams* p, int batc
             hipLaunchKernelGGL(fmha_fwd_d64_bf16_msk0, grid, block, 0, stream, *p);
     }
     return hipGetLastError();
+}
+
+hipError_t run(const FmhaFwdParams* p, int batch, int causal, const Launch& l, void* workspace, int64_t bytes,
+               hipStream_t stream) {
+    switch (l.form) {
+        case -1: return hipErrorInvalidValue;
+        case 0: return hipSuccess;  // nothing to compute
+        case FMHA_FORM_DECODE: return decode_run(p, batch, causal, l.dev.cus, workspace, bytes, stream);
+        case FMHA_FORM_CHUNK: {
+            FmhaChunkArgs c;
+            int64_t need = 0;
+            if (!chunk_plan(p, batch, causal, l.dev.cus, &c, &need)) return hipErrorInvalidValue;
+            c.part = (float*)workspace;
+            return chunk_launch(c, batch, causal, stream);
+        }
+        case FMHA_VARIANT_BALANCED:
+        case FMHA_VARIANT_BALANCED_PAIR: return balanced_launch(p, batch, causal, l, workspace, stream);
+        default: return grid_launch(p, batch, causal, l, stream);
+    }
+}
+
+}  // namespace
+
+extern "C" int fmha_fwd_d64_bf16_balanced_plan(const FmhaFwdParams* p, int batch, int causal, int compute_units,
+                                               int xccs, int force, unsigned short* items, int capacity,
+                                               int* split_from) {
+    if (fmha_fwd_d64_bf16_check(p, batch, causal) != hipSuccess || compute_units < 0 || xccs < 0) return -1;
+    if (force < kPlanAuto || force > kPlanPair) return -1;
+    FmhaBalancedArgs a;
+    if (!balanced_plan(p, batch, causal, compute_units > 0 ? compute_units : device_cus(),
+                       xccs > 0 ? xccs : device_shape().xccs, force, &a, nullptr))
+        return 0;
+    if (items != nullptr)
+        for (int i = 0; i < a.n_items && i < capacity; ++i) items[i] = a.item[i];
+    if (split_from != nullptr) *split_from = a.split_from;
+    return a.n_items;
+}
+
+int64_t fmha_balanced_workspace_size(const FmhaFwdParams* p, int batch, int causal, int variant) {
+    if (fmha_fwd_d64_bf16_check(p, batch, causal) != hipSuccess) return -1;
+    const int order = order_of(variant);
+    if (order < 0) return -1;
+    const int mode = plan_mode(variant & ~kOrderFlags);
+    if (mode < 0) return 0;
+    int64_t bytes = 0;
+    // the same plan (and cache entry) as the launch with this variant
+    const DeviceShape dev = device_shape();
+    if (!balanced_plan(p, batch, causal, dev.cus, plan_xccs(order, dev), mode, nullptr, &bytes)) return 0;
+    return bytes;
+}
+
+extern "C" int64_t fmha_fwd_d64_bf16_workspace_size(const FmhaFwdParams* p, int batch, int causal, int variant) {
+    if (fmha_fwd_d64_bf16_check(p, batch, causal) != hipSuccess) return -1;
+    if (variant == FMHA_VARIANT_AUTO && batch > 0 && p->seqlen_q > 0) {
+        const int64_t cus = device_cus();
+        int64_t bytes = 0;
+        if (takes_decode(p, batch, causal, cus, true, true)) return decode_bytes(p, batch, cus);
+        if (chunk_plan(p, batch, causal, cus, nullptr, &bytes)) return bytes;
+    }
+    return fmha_balanced_workspace_size(p, batch, causal, variant);
+}
+
+extern "C" int fmha_fwd_d64_bf16_form(const FmhaFwdParams* p, int batch, int causal, int variant,
+                                      int64_t workspace_bytes) {
+    if (fmha_fwd_d64_bf16_check(p, batch, causal) != hipSuccess || workspace_bytes < 0) return -1;
+    return decide(p, batch, causal, variant, true, workspace_bytes).form;
+}
+
+extern "C" hipError_t fmha_fwd_d64_bf16_ws(const FmhaFwdParams* p, int batch, int causal, int variant,
+                                           void* workspace, int64_t workspace_bytes, hipStream_t stream) {
+    const hipError_t chk = fmha_fwd_d64_bf16_check(p, batch, causal);
+    if (chk != hipSuccess) return chk;
+    if (plan_mode(variant & ~kOrderFlags) >= 0 &&  // the other variants use no workspace
+        (workspace_bytes < 0 || (workspace == nullptr && workspace_bytes != 0) ||
+         (reinterpret_cast<uintptr_t>(workspace) & 255u)))
+        return hipErrorInvalidValue;
+    return run(p, batch, causal, decide(p, batch, causal, variant, true, workspace_bytes), workspace, workspace_bytes,
+               stream);
+}
+
+extern "C" hipError_t fmha_fwd_d64_bf16_variant(const FmhaFwdParams* p, int batch, int causal, int variant,
+                                                hipStream_t stream) {
+    const hipError_t chk = fmha_fwd_d64_bf16_check(p, batch, causal);
+    if (chk != hipSuccess) return chk;
+    return run(p, batch, causal, decide(p, batch, causal, variant, false, 0), nullptr, 0, stream);
+}
+
+extern "C" int fmha_fwd_d64_bf16_pick_variant(const FmhaFwdParams* p, int batch, int causal, int compute_units) {
+    if (fmha_fwd_d64_bf16_check(p, batch, causal) != hipSuccess || compute_units < 0) return -1;
+    const int64_t cus = compute_units > 0 ? compute_units : device_cus();
+    return pick_form(p, batch, causal, cus);
+}
+
+extern "C" int fmha_fwd_d64_bf16_tile_major(const FmhaFwdParams* p, int batch, int causal) {
+    if (fmha_fwd_d64_bf16_check(p, batch, causal) != hipSuccess) return -1;
+    if (p->seqlen_q == 0 || batch == 0) return 0;  // nothing is launched
+    const DeviceShape dev = device_shape();
+    if (dense_tile_major(p, batch, causal, kOrderAuto, dev)) return 1;
+    // varlen: the compact orders, which only the regular form has
+    if (pick_form(p, batch, causal, dev.cus) != FMHA_VARIANT_REGULAR) return 0;
+    const int o = varlen_order(p, batch, causal, kOrderAuto, dev.cus);
+    return o == kOrderTileMajor ? 1 : o == kOrderSequence ? 2 : 0;
 }
 
 extern "C" hipError_t fmha_fwd_d64_bf16(const FmhaFwdParams* p, int batch, int causal, hipStream_t stream) {

@@ -84,9 +84,9 @@ __global__ void fmha_fwd_d64_bf16_decode_merge_msk1(FmhaDecodeArgs args);
 __global__ void fmha_fwd_d64_bf16_decode_merge_msk0_varlen(FmhaDecodeArgs args);
 __global__ void fmha_fwd_d64_bf16_decode_merge_msk1_varlen(FmhaDecodeArgs args);
 
-// fmha_fwd_d64_bf16_workspace_size for the balanced forms alone (the entry
-// point on the static array splits no decode launch: calls on several streams
-// that needed no scratch must not start to share it).
+// fmha_fwd_d64_bf16_workspace_size for the balanced forms alone: what the entry
+// point on the static array gives a launch (calls on several streams that need
+// no balanced plan must not share it).
 int64_t fmha_balanced_workspace_size(const FmhaFwdParams* p, int batch, int causal, int variant);
 
 // Wide form (see fmha_fwd_kernel.hip): 64 query rows per wave.

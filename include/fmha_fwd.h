@@ -150,12 +150,12 @@ hipError_t fmha_fwd_d64_bf16(const FmhaFwdParams* params, int batch, int causal,
  *                         taking every CU-count-th pair; causal: one block
  *                         per pair of the first half of each (batch, head),
  *                         taking that pair's mirror next
- * The wide form (64 query rows per wave, blocks of 256 rows) has no code of its
- * own either: AUTO launches of dense layouts without an order flag that would run
+ * The wide form (64 query rows per wave, blocks of 256 rows) has no variant code
+ * (fmha_fwd_d64_bf16_form reports it): AUTO launches of dense layouts without an order flag that would run
  * the regular or the pair form take it where its blocks are estimated to fill the
  * compute units better (causal squares: from four blocks per compute unit and
  * 2,560 keys).
- * The decode form has no code of its own: the query heads of a KV head share
+ * Nor has the decode form: the query heads of a KV head share
  * one pass over its keys, whose 32-key steps the waves of a block split, and
  * with a workspace (fmha_fwd_d64_bf16_ws) the blocks too; an order flag keeps
  * the M-tile forms.  In varlen launches it computes the rows the M-tile grid
@@ -250,7 +250,9 @@ int64_t fmha_fwd_d64_bf16_workspace_size(const FmhaFwdParams* params, int batch,
  * until the process ends; a launch whose plan needs more returns
  * hipErrorInvalidValue and launches nothing (the balanced form needs
  * 2 x 34,816 bytes per split M-tile: B1 H2 S40000 causal needs 30,359,552).
- * The decode form runs unsplit here: it uses none of the array.
+ * Only launches for which the balanced form's rule has a plan use the array
+ * (the form they then run may be another that fits in that plan's bytes); all
+ * others, unsplit decode launches among them, use none of it.
  * Calls that overlap in time on one GPU share the array and race; calls in
  * stream order do not (nothing in it needs clearing).  Allocates nothing. */
 #define FMHA_NOALLOC_SCRATCH_BYTES (32 << 20)
@@ -277,8 +279,18 @@ int fmha_fwd_d64_bf16_balanced_plan(const FmhaFwdParams* params, int batch, int 
  * needed).  Returns hipSuccess or hipErrorInvalidValue. */
 hipError_t fmha_fwd_d64_bf16_check(const FmhaFwdParams* params, int batch, int causal);
 
-/* The form FMHA_VARIANT_AUTO resolves to where the decode or wide form does not
- * take the launch, for these arguments on a device with
+/* The form that fmha_fwd_d64_bf16_ws runs for these arguments and workspace size
+ * on the current device (0 bytes: also fmha_fwd_d64_bf16 and _variant), without
+ * launching (this build's own; no counterpart in the reference): a
+ * FMHA_VARIANT_* or FMHA_FORM_* code, 0 when nothing is launched (no batch or no
+ * queries), -1 for rejected arguments. */
+#define FMHA_FORM_DECODE 9 /* forms without a variant code */
+#define FMHA_FORM_CHUNK 10
+#define FMHA_FORM_WIDE 11
+int fmha_fwd_d64_bf16_form(const FmhaFwdParams* params, int batch, int causal, int variant, int64_t workspace_bytes);
+
+/* The M-tile form FMHA_VARIANT_AUTO resolves to where no other takes the
+ * launch (fmha_fwd_d64_bf16_form reports those too), for these arguments on a device with
  * `compute_units` compute units (0 = the current device's count), without
  * launching (this build's own; no counterpart in the reference).  Returns
  * FMHA_VARIANT_REGULAR, _SPLITKV, _PAIR or _SHORT, or -1 for rejected

@@ -1,0 +1,93 @@
+"""The form a launch runs, as the launcher decides it (host only; 256 compute
+units and 8 XCDs where there is no GPU, as on the MI355X)."""
+import random
+
+import pytest
+
+import fmha_native_amd as fmha
+
+AUTO, REF = fmha.VARIANT_AUTO, fmha.VARIANT_REFERENCE_ORDER
+BIG = 1 << 40
+
+
+def params(h, hk, sq, sk, varlen=False):
+    p = fmha.FmhaFwdParams()
+    p.q = p.k = p.v = p.o = 1 << 20
+    p.scale, p.nhead_q, p.nhead_k, p.seqlen_q, p.seqlen_k = 0.18, h, hk, sq, sk
+    for n in "qkvo":
+        for f in ("stride", "nhead_stride", "batch_stride"):
+            setattr(p, f"{f}_{n}", 64)
+    if varlen:
+        p.seqstart_q = p.seqstart_k = 1 << 20
+    return p
+
+
+def form(b, h, hk, sq, sk, causal, ws=0, variant=AUTO, varlen=False):
+    return fmha.FORMS.get(fmha.launch_form(params(h, hk, sq, sk, varlen), b, causal, variant, ws))
+
+
+@pytest.mark.parametrize("b,h,hk,sq,sk,causal,plain,with_ws", [
+    (1, 2, 2, 128, 128, 0, "regular", "regular"),
+    (4, 16, 16, 2048, 2048, 0, "wide", "wide"),
+    (1, 16, 16, 8192, 8192, 1, "pair", "pair"),
+    (1, 2, 2, 40000, 40000, 1, "regular", "balanced"),
+    (128, 16, 16, 128, 128, 0, "short", "short"),
+    (16, 32, 8, 1, 4100, 1, "decode", "decode"),
+    (1, 16, 4, 512, 16384, 1, "decode", "chunk"),
+    (1, 4, 4, 4096, 4096, 0, "splitkv", "chunk"),
+    (1, 8, 8, 512, 512, 0, "decode", "decode"),
+])
+def test_forms_of_common_launches(b, h, hk, sq, sk, causal, plain, with_ws):
+    assert form(b, h, hk, sq, sk, causal) == plain
+    assert form(b, h, hk, sq, sk, causal, BIG) == with_ws
+
+
+def test_named_variants_and_order_flags_keep_their_form():
+    for v in ("regular", "splitkv", "pair", "short", "pair_stream"):
+        for ws in (0, BIG):
+            assert form(2, 8, 8, 1, 4096, 1, ws, fmha.VARIANTS[v]) == v
+            assert form(2, 8, 8, 1, 4096, 1, ws, fmha.VARIANTS[v] | REF) == v
+    for flag in (REF, fmha.VARIANT_TILE_MAJOR_ORDER, fmha.VARIANT_SEQUENCE_ORDER):
+        assert form(4, 16, 16, 2048, 2048, 0, 0, AUTO | flag) == "pair"      # wide without the flag
+        assert form(16, 32, 8, 1, 4100, 1, BIG, AUTO | flag) == "regular"    # decode without it
+        assert form(1, 16, 4, 512, 16384, 1, BIG, AUTO | flag) == "balanced"  # chunk without it
+        assert form(1, 2, 2, 40000, 40000, 1, BIG, AUTO | flag) == "balanced"
+
+
+def test_rejected_and_empty_launches():
+    p = params(2, 2, 40000, 40000)
+    f = lambda v, ws=0, b=1, c=1, q=p: fmha.launch_form(q, b, c, v, ws)
+    for v in (fmha.VARIANT_BALANCED, fmha.VARIANT_BALANCED_PAIR):
+        need = fmha.workspace_size(p, 1, 1, v)
+        assert need > 0 and f(v, need) == v and f(v, need - 1) == -1 and f(v, BIG, c=0) == -1
+        assert f(v, 0, b=0) == 0
+    assert f(4) == f(99) == f(REF | fmha.VARIANT_TILE_MAJOR_ORDER) == f(AUTO, -1) == f(AUTO, 0, c=2) == -1
+    v = params(2, 2, 400, 400, varlen=True)
+    assert f(fmha.VARIANT_PAIR_STREAM, q=v) == f(fmha.VARIANT_PAIR_STREAM, b=0, q=v) == -1
+    assert f(AUTO, b=0) == f(AUTO, q=params(2, 2, 0, 400)) == f(fmha.VARIANT_PAIR, b=0) == 0
+
+
+def test_workspace_and_form_agree():
+    """The bytes workspace_size asks for are those its form needs: one byte
+    less and another form runs (decode: the same, unsplit); none and the
+    launch needs none."""
+    r = random.Random(5)
+    seen = set()
+    for _ in range(3000):
+        h, hk = r.choice([(1, 1), (2, 2), (4, 4), (8, 8), (16, 16), (32, 8), (16, 2), (6, 3)])
+        sq, sk = int(2 ** r.uniform(0, 14)), int(2 ** r.uniform(0, 15))
+        b, causal, varlen = int(2 ** r.uniform(0, 7)), r.randrange(2), r.random() < 0.2
+        p = params(h, hk, sq, sk, varlen)
+        need = fmha.workspace_size(p, b, causal)
+        f = fmha.launch_form(p, b, causal, AUTO, need)
+        tag = (b, h, hk, sq, sk, causal, varlen, need, f)
+        seen.add((f, need > 0))
+        if f in (fmha.FORM_CHUNK, fmha.VARIANT_BALANCED):
+            assert need > 0 and not varlen and need % 34816 == 0, tag
+            assert fmha.launch_form(p, b, causal, AUTO, need - 1) != f, tag
+        elif f != fmha.FORM_DECODE:
+            assert need == 0, tag
+        if need == 0 and f not in (fmha.FORM_DECODE, fmha.FORM_WIDE):
+            assert f == fmha.pick_variant(p, b, causal), tag
+    assert {(fmha.FORM_DECODE, True), (fmha.FORM_DECODE, False), (fmha.FORM_CHUNK, True), (fmha.FORM_WIDE, False),
+            (fmha.VARIANT_BALANCED, True)} <= seen
