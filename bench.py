@@ -196,14 +196,13 @@ def time_problem(prob, steps, warmup, torch, mult=1.0, variant=0):
     torch.cuda.synchronize()
     ref_ms = sum(times) / steps
     hip.destroy([e0, e1])
-    orders = fmha.VARIANT_REFERENCE_ORDER | fmha.VARIANT_TILE_MAJOR_ORDER | fmha.VARIANT_SEQUENCE_ORDER
-    picked = (variant & ~orders) or fmha.pick_variant(p, batch, causal)
-    plain = ", plain heaviest-first table" if variant & fmha.VARIANT_REFERENCE_ORDER else ""
-    form = ("balanced pair" if picked == fmha.VARIANT_BALANCED_PAIR else "balanced") + plain + \
-        " (two launches: items, then the merge of split M-tiles)" if need > 0 else \
-        {v: k for k, v in fmha.VARIANTS.items()}.get(picked, "?")
-    if not variant and need <= 0 and not prob.varlen:  # the launcher's own refinement of the M-tile rule has no code
-        form += " (or the wide or decode form, where the launcher estimates it faster)"
+    picked = fmha.launch_form(p, batch, causal, variant, need)
+    form = fmha.FORMS[picked].replace("_", " ")
+    if picked in (fmha.VARIANT_BALANCED, fmha.VARIANT_BALANCED_PAIR):
+        form += ", plain heaviest-first table" if variant & fmha.VARIANT_REFERENCE_ORDER else ""
+        form += " (two launches: items, then the merge of split M-tiles)"
+    elif need > 0:
+        form += " (two launches: key ranges, then their merge)"
     return {"ms": ms, "wall_ms": wall * 1e3 / steps, "tflops": prob.flops() / (ms * 1e-3) / 1e12, "ramp": ramp,
             "ref_ms": ref_ms, "ref_tflops": prob.flops() / (ref_ms * 1e-3) / 1e12, "host": host, "form": form,
             "workspace_bytes": need}

@@ -56,6 +56,7 @@ def test_chunk_matches_float64(b, h, hk, sq, sk, causal):
     refs = [_f64(q[i], k[i], v[i], causal) for i in range(b)]
     outs = []
     for size in (need, need, need - 1):
+        assert (fmha.launch_form(p, b, causal, fmha.VARIANT_AUTO, size) == fmha.FORM_CHUNK) == (size == need)
         o.fill_(float("nan"))
         lse.fill_(float("nan"))
         fmha.fmha_fwd_d64_bf16_ws(p, b, causal, ws.data_ptr(), size, torch.cuda.current_stream().cuda_stream)

@@ -110,6 +110,7 @@ def test_decode_matches_float64(b, h, hk, sq, sk, causal):
     stream = torch.cuda.current_stream().cuda_stream
     outs = []
     for size in (0, need, need):
+        assert fmha.launch_form(p, b, causal, fmha.VARIANT_AUTO, size) == fmha.FORM_DECODE
         o.fill_(float("nan"))
         lse.fill_(float("nan"))
         fmha.fmha_fwd_d64_bf16_ws(p, b, causal, ws.data_ptr() if size else None, size, stream)
@@ -141,6 +142,7 @@ def test_decode_varlen_matches_float64(causal, bound):
     if bound:
         p.seqlen_k = bound
     for size in (0, fmha.workspace_size(p, len(lk), causal)):
+        assert fmha.launch_form(p, len(lk), causal, fmha.VARIANT_AUTO, size) == fmha.FORM_DECODE
         ws = torch.full((max(size, 256),), 0xFF, dtype=torch.uint8, device="cuda")
         o.fill_(float("nan"))
         lse.fill_(float("nan"))
@@ -178,6 +180,7 @@ def test_decode_varlen_rows_past_the_query_bound(h, hk, lq, lk, bound, causal):
     need = fmha.workspace_size(p, batch, causal)
     ws = torch.full((max(need, 256),), 0xFF, dtype=torch.uint8, device="cuda")
     for size in sorted({0, need}):
+        assert fmha.launch_form(p, batch, causal, fmha.VARIANT_AUTO, size) == fmha.FORM_DECODE
         o.fill_(float("nan"))
         lse.fill_(float("nan"))
         fmha.fmha_fwd_d64_bf16_ws(p, batch, causal, ws.data_ptr() if size else None, size,

@@ -11,6 +11,8 @@ def _run(q, k, v, causal, variant):
     o = torch.full_like(q, float("nan"))
     lse = torch.full(q.shape[:-1], float("nan"), device="cuda")
     p = fmha.params_from_tensors(q, k, v, o, lse)
+    form = fmha.FORM_WIDE if variant == fmha.VARIANT_AUTO else variant
+    assert fmha.launch_form(p, q.shape[0], causal, variant) == form
     fmha.fmha_fwd_d64_bf16(p, q.shape[0], causal, torch.cuda.current_stream().cuda_stream, variant)
     torch.cuda.synchronize()
     return o, lse
