@@ -728,19 +728,27 @@ hipError_t chunk_launch(const FmhaChunkArgs& a, int batch, int causal, hipStream
 //    71 / 65, B64 H8 S256 17.2 / 15.5; k = 3 full B6 H16 S2048 108 / 98, B12 H16
 //    S1000 58 / 52; partial last rounds lose: B3 H16 S2048 (1.5 rounds) 56 / 60,
 //    B9 H16 S900 43.6 / 44.9, B8 H16 S1030 (an odd M-tile) 47.1 / 48.5.
+//    k = 1 is one wave per SIMD against the regular form's two: 3-6 % slower over
+//    490 shapes (H40 1024 x 512 11.7 / 12.4, H32 2048 x 256 8.6 / 9.6; a mask
+//    7-39 %), but where a head's two M-tiles fall on different XCDs (heads go
+//    round robin) and its keys are few, one block reads them once: B26 H6 153 x
+//    848 20.0 / 17.6, B54 H4/1 132 x 1159 27.1 / 24.3, B14 H12 238 x 238 10.5 /
+//    9.4; past 20 key tiles 0.85-1.13x, with 8 heads per XCD round 0.98-1.08x.
 //  * Causal squares: the heaviest-first order levels the blocks from four per CU,
 //    and the waves' different diagonals (up to three tiles of a block's) cost
 //    little from 2,560 keys: H32 S8192 283 / 262, H16 S16384 543 / 501, B12 H32
 //    S3000 519 / 478, B4 H32 S4096 304 / 290; B16 H16 S2048 179 / 178, B16 H16
 //    S1024 56 / 63, H24 S6000 (576 blocks) 122 / 130, H16 S8192 (512) 142 / 155.
-bool takes_wide(const FmhaFwdParams* p, int batch, int causal, int form, int64_t cus) {
+bool takes_wide(const FmhaFwdParams* p, int batch, int causal, int form, const DeviceShape& d) {
     if (p->seqstart_q != nullptr || p->seqlen_k <= 0) return false;
+    const int64_t cus = d.cus;
     if (form != FMHA_VARIANT_REGULAR && form != FMHA_VARIANT_PAIR) return false;
     const int m_tiles = (p->seqlen_q + kM0 - 1) / kM0;
     const int longest = mtile_tiles(p, causal, m_tiles - 1);
     const int lightest = mtile_tiles(p, causal, std::min(1, m_tiles - 1));
     const int64_t wide = pair_blocks(p, batch), regular = grid_blocks(p, batch);
     if (4 * (int64_t)lightest < 3 * (int64_t)longest) return wide >= 4 * cus && longest >= 40;
+    if (wide <= cus && (causal || m_tiles != 2 || p->nhead_q % d.xccs == 0 || longest > 20)) return false;
     auto us = [cus](int64_t blocks, double two, double one) {
         const int64_t k = (blocks + cus - 1) / cus;  // blocks of the fullest CU
         return two * (double)(k / 2) + one * (double)(k % 2);
@@ -819,7 +827,7 @@ Launch decide(const FmhaFwdParams* p, int batch, int causal, int variant, bool w
         l.plan_auto = bytes > 0 && balanced_plan(p, batch, causal, cus, plan_xccs(l.order, l.dev), kPlanAuto, nullptr,
                                                  &need) && need <= bytes;
         l.form = l.plan_auto ? FMHA_VARIANT_BALANCED : pick_form(p, batch, causal, cus);
-        if (!l.plan_auto && l.order == kOrderAuto && takes_wide(p, batch, causal, l.form, cus))
+        if (!l.plan_auto && l.order == kOrderAuto && takes_wide(p, batch, causal, l.form, l.dev))
             l.form = FMHA_FORM_WIDE;
         return l;
     }

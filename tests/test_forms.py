@@ -91,3 +91,17 @@ def test_workspace_and_form_agree():
             assert f == fmha.pick_variant(p, b, causal), tag
     assert {(fmha.FORM_DECODE, True), (fmha.FORM_DECODE, False), (fmha.FORM_CHUNK, True), (fmha.FORM_WIDE, False),
             (fmha.VARIANT_BALANCED, True)} <= seen
+
+
+@pytest.mark.parametrize("b,h,hk,sq,sk,causal,wide", [
+    (64, 8, 8, 256, 256, 0, True), (4, 16, 16, 2048, 2048, 0, True), (12, 16, 16, 1000, 1000, 0, True),  # two or more
+    # at most one 256-row block per compute unit: one wave per SIMD
+    (1, 40, 40, 1024, 512, 0, False), (1, 32, 32, 2048, 256, 0, False), (1, 64, 64, 767, 512, 0, False),
+    (3, 24, 24, 445, 870, 1, False), (2, 16, 4, 1918, 1918, 0, False), (20, 4, 1, 389, 479, 1, False),
+    (32, 8, 8, 132, 76, 0, False), (18, 8, 2, 155, 324, 0, False),
+    # ... but a head's two M-tiles would run on two XCDs and its keys are few
+    (26, 6, 6, 153, 848, 0, True), (54, 4, 1, 132, 1159, 0, True), (14, 12, 12, 238, 238, 0, True),
+    (14, 12, 12, 238, 1281, 0, False), (14, 12, 12, 238, 238, 1, False), (9, 6, 6, 546, 135, 0, False),
+])
+def test_wide_rule(b, h, hk, sq, sk, causal, wide):
+    assert (form(b, h, hk, sq, sk, causal) == "wide") == wide
