@@ -429,7 +429,7 @@ bool balanced_plan_build(const FmhaFwdParams* p, int batch, int causal, int64_t 
 
 // ---- chunk form (kModeChunk in fmha_fwd_kernel.hip) ----
 //
-// Dense launches of at most 0.6 M-tiles per compute unit, with a workspace.
+// Dense launches of at most 5/8 M-tile per compute unit, with a workspace.
 // What bounds them is one block's chain of key tiles (split-KV halves it,
 // the balanced form too), so M-tiles of more than `tiles` key tiles are cut
 // into equal chunks that run as blocks of their own, all resident at once, and
@@ -437,6 +437,7 @@ bool balanced_plan_build(const FmhaFwdParams* p, int batch, int causal, int64_t 
 // shapes (16-144 M-tiles of 11-313 key tiles, 12 chunk lengths each), a launch
 // of I chunk blocks, the longest of w tiles, at most c per M-tile, takes
 //     6.1 + k (w + 1) + 0.0127 I + 0.3 c   us,
+// (w over all M-tiles: causal ones just below the chunk length stay whole),
 // k = 0.55 up to one block per CU and 0.9 up to two (rms error 8 %): shorter
 // chunks trade the chain against the partials' traffic and the merge's.  The
 // forms without chunks take 9.5 + 0.275 n us (balanced), 6 + 0.435 n
@@ -445,7 +446,8 @@ bool balanced_plan_build(const FmhaFwdParams* p, int batch, int causal, int64_t 
 // the other form's.  Start / chunks: B1 H16 512 x 16384 causal 78 / 46 us,
 // H16 100 x 8192 43 / 18, H2 S4096 causal 26 / 17, H1 S16384 causal 80 / 53,
 // H4 S4096 34 / 29, H6 S2500 23.7 / 21.5; H16 S1024 (128 M-tiles of 16 tiles)
-// stays regular, 12.5 / 14.
+// stays regular, 12.5 / 14, and H72 256 x 2048 causal (M-tiles of 30 and 32
+// tiles: cutting the longer ones alone leaves 30) split-KV, 20.3 / 26.0.
 struct ChunkChoice {
     int tiles;  // key tiles per chunk
     double us;  // estimate
@@ -462,6 +464,15 @@ int64_t chunk_items(const FmhaFwdParams* p, int causal, int m_tiles, int64_t hb,
     for (int mt = 0; mt < m_tiles; ++mt) n += chunk_count(causal_ntiles(p, mt), tiles);
     return hb * n;
 }
+// Key tiles of the longest chunk.
+int chunk_longest(const FmhaFwdParams* p, int causal, int m_tiles, int tiles) {
+    int w = 0;
+    for (int mt = causal ? 0 : m_tiles - 1; mt < m_tiles; ++mt) {
+        const int n = mtile_tiles(p, causal, mt), c = std::min(FMHA_CHUNK_MAX_CHUNKS, chunk_count(n, tiles));
+        w = std::max(w, (n + c - 1) / c);
+    }
+    return w;
+}
 // The chunk length for at most `slots` blocks at k us per tile.
 ChunkChoice chunk_choice(const FmhaFwdParams* p, int causal, int m_tiles, int64_t hb, int longest, double total,
                          int64_t slots, double k) {
@@ -477,7 +488,7 @@ ChunkChoice chunk_choice(const FmhaFwdParams* p, int causal, int m_tiles, int64_
     }
     if (lo >= longest) return {0, 0.0};
     const int c = std::min(FMHA_CHUNK_MAX_CHUNKS, chunk_count(longest, lo));
-    const double w = (longest + c - 1) / c;
+    const double w = chunk_longest(p, causal, m_tiles, lo);
     return {lo, 6.1 + k * (w + 1.0) + 0.0127 * (double)chunk_items(p, causal, m_tiles, hb, lo) + 0.3 * c};
 }
 // The M-tile forms' estimate for launches of at most one block per CU, and

@@ -213,7 +213,7 @@ hipError_t fmha_fwd_d64_bf16_variant(const FmhaFwdParams* params, int batch, int
  *            the compute units and seqlen_k > 1280: each block's fp32 partial
  *            goes to the workspace and a second launch merges them, unsplit
  *            if the workspace is too small; the chunk form for dense launches
- *            of at most 0.6 M-tiles per compute unit whose long M-tiles it
+ *            of at most 5/8 M-tile per compute unit whose long M-tiles it
  *            estimates faster in key chunks: each chunk's fp32 partial goes to
  *            the workspace and a second launch merges them; without an order
  *            flag; else what fmha_fwd_d64_bf16 picks),

@@ -105,3 +105,15 @@ def test_workspace_and_form_agree():
 ])
 def test_wide_rule(b, h, hk, sq, sk, causal, wide):
     assert (form(b, h, hk, sq, sk, causal) == "wide") == wide
+
+
+@pytest.mark.parametrize("b,h,sq,sk,causal,chunk", [
+    (1, 16, 512, 16384, 1, True), (1, 4, 4096, 4096, 0, True), (1, 2, 4096, 4096, 1, True), (2, 24, 124, 9467, 0, True),
+    # causal M-tiles of nearly one length: a chunk length that cuts the longest
+    # ones alone leaves the others whole, as long as they were
+    (1, 72, 256, 2048, 1, False), (1, 80, 256, 2048, 1, False), (1, 40, 512, 2048, 1, False),
+    (1, 32, 640, 2048, 1, False), (2, 24, 298, 5399, 1, False),
+    (1, 16, 1024, 1024, 0, False), (5, 32, 128, 9000, 0, True), (161, 1, 128, 9000, 0, False),  # 5/8 per CU: 160
+])
+def test_chunk_form_rule(b, h, sq, sk, causal, chunk):
+    assert (form(b, h, h, sq, sk, causal, BIG) == "chunk") == chunk
