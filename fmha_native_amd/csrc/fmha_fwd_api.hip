@@ -12,6 +12,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
+#include <numeric>
 
 #include "fmha_fwd.h"
 #include "fmha_internal.h"
@@ -570,7 +571,11 @@ int decode_chunks(const FmhaFwdParams* p, int batch, int64_t cus) {
 //    block's chain of key tiles, which the decode form splits over eight waves:
 //    5.9 + 0.65 us per 256-key step (0.8 above half a block per CU, where two
 //    waves share a SIMD's matrix core with nothing left over) + 3.2 for the
-//    merge of a split launch, against the estimates of the other forms.  H8
+//    merge of a split launch, and no less than 4 us + K and V once at 5.4 TB/s or
+//    once per XCD that a head's row tiles fall on (heads and chunks go round
+//    robin) at 7 TB/s (rms error 10 % over 880 launches above 10 us, 21 % without
+//    it: B14 H6 40 x 7106 causal took 45.0, the chain's estimate 28.3, the balanced
+//    form 41.8), against the estimates of the other forms.  H8
 //    S512 8.0 / 6.9, H4 S1024 12.3 / 7.8, H8 S1024 causal 12.9 / 7.9, H2 S2048
 //    19.6 / 10.8, H4 256 x 8192 17.4 / 12.8, B8 H16/2 64 x 1000 13.2 / 8.3, H16
 //    100 x 8192 17.9 / 14.5 (chunks / decode); up to 256 keys both take one
@@ -580,12 +585,11 @@ int decode_chunks(const FmhaFwdParams* p, int batch, int64_t cus) {
 // `split`: a workspace holds the split launch's partials; `workspace`: there
 // is one at all (the balanced and chunk forms' estimates count).
 struct DecodeAsk {
-    int seqlen_q, seqlen_k, nhead_q, nhead_k, batch, causal, split, workspace;
-    int64_t cus;
+    int seqlen_q, seqlen_k, nhead_q, nhead_k, batch, causal, split, workspace, cus, xccs;
     bool operator==(const DecodeAsk& o) const {
         return seqlen_q == o.seqlen_q && seqlen_k == o.seqlen_k && nhead_q == o.nhead_q && nhead_k == o.nhead_k &&
                batch == o.batch && causal == o.causal && split == o.split && workspace == o.workspace &&
-               cus == o.cus;
+               cus == o.cus && xccs == o.xccs;
     }
 };
 bool decode_faster(const FmhaFwdParams* p, const DecodeAsk& a) {
@@ -593,23 +597,28 @@ bool decode_faster(const FmhaFwdParams* p, const DecodeAsk& a) {
     if (items > a.cus) return false;
     const int chunks = a.split ? decode_chunks(p, a.batch, a.cus) : 1;
     const int steps = (p->seqlen_k + FMHA_DECODE_KEY_STEP - 1) / FMHA_DECODE_KEY_STEP;
-    const double us =
-        5.9 + (2 * items > a.cus ? 0.8 : 0.65) * ((steps + chunks - 1) / chunks) + (chunks > 1 ? 3.2 : 0.0);
+    const int per = (steps + chunks - 1) / chunks, n_chunks = (steps + per - 1) / per;
+    const int64_t row_tiles = (decode_rows(p) + FMHA_DECODE_ROWS - 1) / FMHA_DECODE_ROWS;
+    const int64_t copies = std::min<int64_t>(row_tiles, a.xccs / std::gcd(p->nhead_k * n_chunks, a.xccs));
+    const double kv = 256e-6 * a.batch * p->nhead_k * (double)p->seqlen_k;  // MB
+    const double us = std::max(5.9 + (2 * items > a.cus ? 0.8 : 0.65) * per,
+                               4.0 + std::max(kv / 5.4, kv * (double)copies / 7.0)) + (chunks > 1 ? 3.2 : 0.0);
     return us < 0.97 * mtile_us(p, a.batch, a.causal, a.cus, a.workspace != 0).us;
 }
-bool takes_decode(const FmhaFwdParams* p, int batch, int causal, int64_t cus, bool split, bool workspace) {
+bool takes_decode(const FmhaFwdParams* p, int batch, int causal, const DeviceShape& d, bool split, bool workspace) {
     if (p->seqlen_k < 128) return false;
     if (decode_rows(p) <= 128 && (p->seqlen_q <= 32 || (p->seqlen_q <= 64 && p->seqlen_k >= 1024))) return true;
     if (p->seqstart_q != nullptr) return false;
     // the estimates walk the M-tiles: a thread's last answers with and without
     // a workspace are kept (they depend on the shape only)
     struct Kept {
-        DecodeAsk ask{-1, -1, -1, -1, -1, -1, -1, -1, -1};
+        DecodeAsk ask{-1, -1, -1, -1, -1, -1, -1, -1, -1, -1};
         bool answer = false;
     };
     thread_local Kept kept[2];
     Kept& last = kept[workspace ? 1 : 0];
-    const DecodeAsk ask{p->seqlen_q, p->seqlen_k, p->nhead_q, p->nhead_k, batch, causal, split, workspace, cus};
+    const DecodeAsk ask{p->seqlen_q, p->seqlen_k, p->nhead_q, p->nhead_k, batch, causal,
+                        split, workspace, d.cus, d.xccs};
     if (!(ask == last.ask)) {
         last.answer = decode_faster(p, ask);
         last.ask = ask;
@@ -825,7 +834,7 @@ Launch decide(const FmhaFwdParams* p, int batch, int causal, int variant, bool w
     int64_t need = 0;
     if (v == FMHA_VARIANT_AUTO) {
         if (l.order == kOrderAuto) {
-            if (takes_decode(p, batch, causal, cus, decode_bytes(p, batch, cus) <= bytes, bytes > 0)) {
+            if (takes_decode(p, batch, causal, l.dev, decode_bytes(p, batch, cus) <= bytes, bytes > 0)) {
                 l.form = FMHA_FORM_DECODE;
                 return l;
             }
@@ -1034,10 +1043,10 @@ int64_t fmha_balanced_workspace_size(const FmhaFwdParams* p, int batch, int caus
 extern "C" int64_t fmha_fwd_d64_bf16_workspace_size(const FmhaFwdParams* p, int batch, int causal, int variant) {
     if (fmha_fwd_d64_bf16_check(p, batch, causal) != hipSuccess) return -1;
     if (variant == FMHA_VARIANT_AUTO && batch > 0 && p->seqlen_q > 0) {
-        const int64_t cus = device_cus();
+        const DeviceShape dev = device_shape();
         int64_t bytes = 0;
-        if (takes_decode(p, batch, causal, cus, true, true)) return decode_bytes(p, batch, cus);
-        if (chunk_plan(p, batch, causal, cus, nullptr, &bytes)) return bytes;
+        if (takes_decode(p, batch, causal, dev, true, true)) return decode_bytes(p, batch, dev.cus);
+        if (chunk_plan(p, batch, causal, dev.cus, nullptr, &bytes)) return bytes;
     }
     return fmha_balanced_workspace_size(p, batch, causal, variant);
 }

@@ -117,3 +117,15 @@ def test_wide_rule(b, h, hk, sq, sk, causal, wide):
 ])
 def test_chunk_form_rule(b, h, sq, sk, causal, chunk):
     assert (form(b, h, h, sq, sk, causal, BIG) == "chunk") == chunk
+
+
+@pytest.mark.parametrize("b,h,hk,sq,sk,causal,ws,expect", [
+    # every row tile of a head on an XCD of its own: K and V come once per tile
+    (7, 6, 6, 165, 5698, 1, BIG, "chunk"), (8, 12, 12, 66, 19520, 1, BIG, "chunk"),
+    (14, 2, 2, 83, 14968, 0, BIG, "chunk"), (10, 3, 3, 116, 10835, 0, BIG, "chunk"),
+    # the chain of key steps bounds these
+    (1, 8, 8, 512, 512, 0, 0, "decode"), (1, 4, 4, 256, 8192, 0, BIG, "decode"), (1, 2, 2, 2048, 2048, 0, BIG, "decode"),
+    (8, 16, 2, 64, 1000, 0, BIG, "decode"),
+])
+def test_decode_estimate_counts_the_memory(b, h, hk, sq, sk, causal, ws, expect):
+    assert form(b, h, hk, sq, sk, causal, ws) == expect
