@@ -560,13 +560,15 @@ int decode_chunks(const FmhaFwdParams* p, int batch, int64_t cus) {
 }
 // Whether a launch runs it: the automatic choice without an order flag (those
 // ask for the M-tile grid); the bounds steer varlen launches.  Two regions:
-//  * decode proper, at most 32 queries (64 from 1024 keys) and 128 packed
-//    rows, bound by the K/V stream.  M-tile forms / decode, us, one box (dense
-//    caches, LSE): B16 H32/8 1 x 4100 82 / 28, B1 H32/8 1 x 32768 312 / 18, B2
-//    H16/2 16 x 16384 77 / 13, B64 H16/16 1 x 128 11.5 / 10.8, B16 H16/16 64 x
-//    4096 62 / 53; past 32 queries short key ranges lose (B64 H16 64 x 200
-//    17 / 22) and past 64 the M-tile forms win (B16 H16 128 x 4096 64 / 87: four
-//    row tiles re-read K and V).
+//  * decode proper, at most 32 queries and 128 packed rows, bound by the K/V
+//    stream.  M-tile forms / decode, us, one box (dense caches, LSE): B16 H32/8
+//    1 x 4100 82 / 28, B1 H32/8 1 x 32768 312 / 18, B2 H16/2 16 x 16384 77 / 13,
+//    B64 H16/16 1 x 128 11.5 / 10.8.  Packed sequences of up to 64 queries too,
+//    from 1024 keys and at most one row tile per compute unit (0.17-1.02x over
+//    35 launches).  Past 32 queries a head has two row tiles that each walk its
+//    keys, and past one round the M-tile forms are ahead (their waves without
+//    rows cost nothing): dense B32 H16/16 64 x 1024 29.5 / 33.0, B76 H6 64 x 1787
+//    causal 42.8 / 62.0, packed 0.77-1.56x over 24 launches.
 //  * dense launches of at most one 32-row tile per compute unit, bound by one
 //    block's chain of key tiles, which the decode form splits over eight waves:
 //    5.9 + 0.65 us per 256-key step (0.8 above half a block per CU, where two
@@ -607,8 +609,9 @@ bool decode_faster(const FmhaFwdParams* p, const DecodeAsk& a) {
 }
 bool takes_decode(const FmhaFwdParams* p, int batch, int causal, const DeviceShape& d, bool split, bool workspace) {
     if (p->seqlen_k < 128) return false;
-    if (decode_rows(p) <= 128 && (p->seqlen_q <= 32 || (p->seqlen_q <= 64 && p->seqlen_k >= 1024))) return true;
-    if (p->seqstart_q != nullptr) return false;
+    if (decode_rows(p) <= 128 && p->seqlen_q <= 32) return true;
+    if (p->seqstart_q != nullptr)
+        return decode_rows(p) <= 128 && p->seqlen_q <= 64 && p->seqlen_k >= 1024 && decode_items(p, batch) <= d.cus;
     // the estimates walk the M-tiles: a thread's last answers with and without
     // a workspace are kept (they depend on the shape only)
     struct Kept {

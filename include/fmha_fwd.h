@@ -117,11 +117,12 @@ hipError_t fmha_fwd_d64_bf16(const FmhaFwdParams* params, int batch, int causal,
 /* The same launch with the kernel form chosen by the caller (this build's
  * own; no counterpart in the reference):
  *   FMHA_VARIANT_AUTO     what fmha_fwd_d64_bf16() picks: the decode form (below)
- *                         from 128 keys on for at most 32 queries (64 from
- *                         1024 keys on) and 128 rows per KV head (nhead_q /
- *                         nhead_k x seqlen_q), and for dense launches of at most
- *                         CUs x 32 such rows in all where it is estimated
- *                         faster; short for
+ *                         from 128 keys on for at most 32 queries and 128 rows
+ *                         per KV head (nhead_q / nhead_k x seqlen_q; varlen: 64
+ *                         queries from 1024 keys on and at most one 32-row tile
+ *                         of a KV head per compute unit), and for dense
+ *                         launches of at most CUs x 32 such rows in all where it
+ *                         is estimated faster; short for
  *                         launches with seqlen_k <= 192 and at least
  *                         2 x CUs x 128 query rows (batch x nhead_q x
  *                         seqlen_q; varlen: the bounds), or causal with

@@ -129,3 +129,17 @@ def test_chunk_form_rule(b, h, sq, sk, causal, chunk):
 ])
 def test_decode_estimate_counts_the_memory(b, h, hk, sq, sk, causal, ws, expect):
     assert form(b, h, hk, sq, sk, causal, ws) == expect
+
+
+@pytest.mark.parametrize("b,h,hk,sq,sk,causal,varlen,decode", [
+    (16, 32, 8, 1, 4100, 1, False, True), (512, 16, 16, 8, 1000, 0, False, True), (16, 8, 8, 32, 2000, 1, True, True),
+    (4, 16, 16, 48, 2000, 0, False, True), (4, 16, 16, 48, 2000, 0, True, True),  # two row tiles, within one round
+    # two row tiles per head, more than one per compute unit
+    (32, 16, 16, 48, 1024, 0, False, False), (76, 6, 6, 64, 1787, 1, False, False), (100, 2, 2, 48, 5550, 1, False, False),
+    (58, 4, 4, 52, 7077, 1, False, False), (32, 32, 16, 64, 2048, 1, False, False),
+    (32, 16, 16, 48, 1024, 0, True, False), (100, 2, 2, 48, 5550, 1, True, False),
+    (4, 16, 16, 48, 900, 0, True, False),
+])
+def test_decode_rule_past_32_queries(b, h, hk, sq, sk, causal, varlen, decode):
+    for ws in (0, BIG):
+        assert (form(b, h, hk, sq, sk, causal, ws, varlen=varlen) == "decode") == decode
