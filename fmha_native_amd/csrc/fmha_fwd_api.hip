@@ -568,7 +568,12 @@ int decode_chunks(const FmhaFwdParams* p, int batch, int64_t cus) {
 //    35 launches).  Past 32 queries a head has two row tiles that each walk its
 //    keys, and past one round the M-tile forms are ahead (their waves without
 //    rows cost nothing): dense B32 H16/16 64 x 1024 29.5 / 33.0, B76 H6 64 x 1787
-//    causal 42.8 / 62.0, packed 0.77-1.56x over 24 launches.
+//    causal 42.8 / 62.0, packed 0.77-1.56x over 24 launches.  Where the short form
+//    would run (two blocks' worth of query rows per compute unit, few keys: both
+//    compute-bound) it takes about 1.2 x row tiles / query heads of a KV head
+//    times as long: B128 H16/16 32 x 128 18.1 / 24.1, one head per KV head
+//    1.05-1.47x over 33 launches, four 0.3-0.7x up to 64 rows and 0.8-1.2x at
+//    128, eight 0.17-0.65x.
 //  * dense launches of at most one 32-row tile per compute unit, bound by one
 //    block's chain of key tiles, which the decode form splits over eight waves:
 //    5.9 + 0.65 us per 256-key step (0.8 above half a block per CU, where two
@@ -609,7 +614,10 @@ bool decode_faster(const FmhaFwdParams* p, const DecodeAsk& a) {
 }
 bool takes_decode(const FmhaFwdParams* p, int batch, int causal, const DeviceShape& d, bool split, bool workspace) {
     if (p->seqlen_k < 128) return false;
-    if (decode_rows(p) <= 128 && p->seqlen_q <= 32) return true;
+    if (decode_rows(p) <= 128 && p->seqlen_q <= 32) {
+        const int64_t tiles = (decode_rows(p) + FMHA_DECODE_ROWS - 1) / FMHA_DECODE_ROWS;
+        return pick_form(p, batch, causal, d.cus) != FMHA_VARIANT_SHORT || 4 * tiles <= 3 * (p->nhead_q / p->nhead_k);
+    }
     if (p->seqstart_q != nullptr)
         return decode_rows(p) <= 128 && p->seqlen_q <= 64 && p->seqlen_k >= 1024 && decode_items(p, batch) <= d.cus;
     // the estimates walk the M-tiles: a thread's last answers with and without

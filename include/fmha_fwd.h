@@ -118,7 +118,9 @@ hipError_t fmha_fwd_d64_bf16(const FmhaFwdParams* params, int batch, int causal,
  * own; no counterpart in the reference):
  *   FMHA_VARIANT_AUTO     what fmha_fwd_d64_bf16() picks: the decode form (below)
  *                         from 128 keys on for at most 32 queries and 128 rows
- *                         per KV head (nhead_q / nhead_k x seqlen_q; varlen: 64
+ *                         per KV head (nhead_q / nhead_k x seqlen_q; where the
+ *                         short form's rule holds too, only for at most 3/4 of
+ *                         a 32-row tile per query head; varlen: 64
  *                         queries from 1024 keys on and at most one 32-row tile
  *                         of a KV head per compute unit), and for dense
  *                         launches of at most CUs x 32 such rows in all where it

@@ -143,3 +143,14 @@ def test_decode_estimate_counts_the_memory(b, h, hk, sq, sk, causal, ws, expect)
 def test_decode_rule_past_32_queries(b, h, hk, sq, sk, causal, varlen, decode):
     for ws in (0, BIG):
         assert (form(b, h, hk, sq, sk, causal, ws, varlen=varlen) == "decode") == decode
+
+
+@pytest.mark.parametrize("varlen", [False, True])
+@pytest.mark.parametrize("b,h,hk,sq,sk,causal,expect", [
+    (128, 16, 16, 32, 128, 0, "short"), (128, 16, 16, 32, 192, 1, "short"), (512, 16, 16, 8, 130, 0, "short"),
+    (600, 16, 16, 32, 380, 1, "short"), (200, 32, 8, 32, 150, 0, "short"),  # four row tiles for four heads
+    (400, 32, 8, 24, 150, 0, "decode"), (400, 32, 8, 16, 150, 0, "decode"), (600, 64, 8, 16, 150, 0, "decode"),
+    (128, 16, 16, 31, 128, 0, "decode"), (128, 16, 16, 32, 193, 0, "decode"),  # not the short form's
+])
+def test_decode_leaves_the_short_form(b, h, hk, sq, sk, causal, expect, varlen):
+    assert form(b, h, hk, sq, sk, causal, varlen=varlen) == expect
