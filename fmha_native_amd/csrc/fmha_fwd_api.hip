@@ -613,7 +613,8 @@ bool decode_faster(const FmhaFwdParams* p, const DecodeAsk& a) {
     return us < 0.97 * mtile_us(p, a.batch, a.causal, a.cus, a.workspace != 0).us;
 }
 bool takes_decode(const FmhaFwdParams* p, int batch, int causal, const DeviceShape& d, bool split, bool workspace) {
-    if (p->seqlen_k < 128) return false;
+    // a grid holds fewer than 2^32 threads, and a decode block up to 512
+    if (p->seqlen_k < 128 || p->nhead_k > (int)(UINT32_MAX / 512)) return false;
     if (decode_rows(p) <= 128 && p->seqlen_q <= 32) {
         const int64_t tiles = (decode_rows(p) + FMHA_DECODE_ROWS - 1) / FMHA_DECODE_ROWS;
         return pick_form(p, batch, causal, d.cus) != FMHA_VARIANT_SHORT || 4 * tiles <= 3 * (p->nhead_q / p->nhead_k);

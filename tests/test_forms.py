@@ -154,3 +154,14 @@ def test_decode_rule_past_32_queries(b, h, hk, sq, sk, causal, varlen, decode):
 ])
 def test_decode_leaves_the_short_form(b, h, hk, sq, sk, causal, expect, varlen):
     assert form(b, h, hk, sq, sk, causal, varlen=varlen) == expect
+
+
+@pytest.mark.parametrize("varlen", [False, True])
+def test_decode_grid_stays_within_the_launch_limit(varlen):
+    """A grid holds fewer than 2^32 threads; eight-wave decode blocks reach it
+    at half the heads the M-tile grid takes (K and V of all heads may be one:
+    head stride 0)."""
+    limit = (1 << 32) // 512
+    assert form(1, limit - 1, limit - 1, 1, 4096, 0, varlen=varlen) == "decode"
+    assert form(1, limit + 1, limit + 1, 1, 4096, 0, varlen=varlen) == "regular"
+    assert form(1, 2 * limit - 2, limit - 1, 1, 4096, 0, varlen=varlen) == "decode"
