@@ -538,8 +538,10 @@ __device__ __forceinline__ void fwd_mtile(const FmhaFwdParams& p, int b, int h, 
     // of the ring and passes the barriers, and computes nothing (the causal
     // entries get there through nlive).  The other blocks of the CU take its
     // issue slots: B8 H16 S1030 50.6 -> 49.3 us, B6 H16 S1100 causal 25.9 ->
-    // 25.2, 64 packed sequences of 16-640 tokens H12 49.2 -> 47.3.
-    if (!kCausal && ntg > 0 && wrow0 >= sq) {
+    // 25.2, 64 packed sequences of 16-640 tokens H12 49.2 -> 47.3.  The path lies
+    // behind the others' code and ends there: inline before it, the instruction
+    // fetch past it cost every short dense launch ~0.3 us.
+    if (__builtin_expect(!kCausal && ntg > 0 && wrow0 >= sq, 0)) {
         issue_k(0, P0{});
         issue_k(1, P1{});
         issue_v(0, P0{});
@@ -559,6 +561,7 @@ __device__ __forceinline__ void fwd_mtile(const FmhaFwdParams& p, int b, int h, 
         }
         vmcnt_wait<0>();
         ring_barrier();  // the other waves' last GEMM1 barrier
+        if constexpr (!kSplitKV) return;  // nothing to store (split-KV: a group barrier follows)
     } else if (ntg > 0) {
         // prologue: Q, then K0 K1 V0 K2 V1 K3 in flight; GEMM0 of tile 0 once
         // Q and K0 landed
@@ -1899,7 +1902,10 @@ __device__ __forceinline__ void fwd_wide(const FmhaFwdParams& p, int b, int h, i
         const int lt = last_key < 0 || wrow0 >= sq ? 0 : last_key / kTileN + 1;
         nlive = max(1, min(ntiles, lt));
     }
-    if (!kCausal && ntiles > 0 && wrow0 >= sq) {  // no rows: the ring only, as in fwd_mtile
+    // no rows: the ring only, as in fwd_mtile (moved behind the others' code it
+    // changes their registers: B4 H16 S2048 68.0 -> 68.4 us, and these launches are
+    // long beside an instruction fetch)
+    if (!kCausal && ntiles > 0 && wrow0 >= sq) {
         issue_k(0, P0{});
         issue_k(1, P1{});
         issue_v(0, P0{});

@@ -149,3 +149,19 @@ def test_short_entries(asm):
         loads = [x for x in ins[:first] if x.startswith("buffer_load_dwordx4")]
         assert sorted("L" if x.endswith(" lds") else "R" for x in loads) == ["L"] * 4 + ["R"] * 4, (name, loads)
         assert all(since == 0 for _, since in _prefetch_waits(body)), name
+
+
+def test_rowless_path_lies_behind_the_others(asm):
+    """Dense entries: the code of waves whose rows are all past the sequence
+    (ring barriers without an MFMA) is not in the way of the others, who would
+    fetch past it on every launch: between the first two barriers in code order
+    lies GEMM0 of the first tile."""
+    seen = 0
+    for name, body in _functions(asm).items():
+        if "msk0" not in name or any(x in name for x in ("merge", "short", "stream", "wide")):
+            continue
+        seen += 1
+        ins = [ln.strip() for ln in body.splitlines() if ln.strip() and not ln.strip().startswith((";", "."))]
+        bars = [i for i, x in enumerate(ins) if x.startswith("s_barrier")]
+        assert any(x.startswith("v_mfma") for x in ins[bars[0]:bars[1]]), name
+    assert seen == 7  # regular, split-KV and pair, each also varlen; chunk
