@@ -765,7 +765,8 @@ hipError_t chunk_launch(const FmhaChunkArgs& a, int batch, int causal, hipStream
 //    7-39 %), but where a head's two M-tiles fall on different XCDs (heads go
 //    round robin) and its keys are few, one block reads them once: B26 H6 153 x
 //    848 20.0 / 17.6, B54 H4/1 132 x 1159 27.1 / 24.3, B14 H12 238 x 238 10.5 /
-//    9.4; past 20 key tiles 0.85-1.13x, with 8 heads per XCD round 0.98-1.08x.
+//    9.4; past 20 key tiles 0.86-1.10x, up to two 0.84-1.07x (H129 256 x 64 5.7 /
+//    6.1), where the heads divide by the XCDs 0.95-1.12x.
 //  * Causal squares: the heaviest-first order levels the blocks from four per CU,
 //    and the waves' different diagonals (up to three tiles of a block's) cost
 //    little from 2,560 keys: H32 S8192 283 / 262, H16 S16384 543 / 501, B12 H32
@@ -780,7 +781,8 @@ bool takes_wide(const FmhaFwdParams* p, int batch, int causal, int form, const D
     const int lightest = mtile_tiles(p, causal, std::min(1, m_tiles - 1));
     const int64_t wide = pair_blocks(p, batch), regular = grid_blocks(p, batch);
     if (4 * (int64_t)lightest < 3 * (int64_t)longest) return wide >= 4 * cus && longest >= 40;
-    if (wide <= cus && (causal || m_tiles != 2 || p->nhead_q % d.xccs == 0 || longest > 20)) return false;
+    if (wide <= cus && (causal || m_tiles != 2 || p->nhead_q % d.xccs == 0 || longest < 3 || longest > 20))
+        return false;
     auto us = [cus](int64_t blocks, double two, double one) {
         const int64_t k = (blocks + cus - 1) / cus;  // blocks of the fullest CU
         return two * (double)(k / 2) + one * (double)(k % 2);

@@ -101,7 +101,7 @@ def test_workspace_and_form_agree():
     (32, 8, 8, 132, 76, 0, False), (18, 8, 2, 155, 324, 0, False),
     # ... but a head's two M-tiles would run on two XCDs and its keys are few
     (26, 6, 6, 153, 848, 0, True), (54, 4, 1, 132, 1159, 0, True), (14, 12, 12, 238, 238, 0, True),
-    (14, 12, 12, 238, 1281, 0, False), (14, 12, 12, 238, 238, 1, False), (9, 6, 6, 546, 135, 0, False),
+    (14, 12, 12, 238, 1281, 0, False), (1, 129, 129, 256, 64, 0, False), (14, 12, 12, 238, 238, 1, False), (9, 6, 6, 546, 135, 0, False),
 ])
 def test_wide_rule(b, h, hk, sq, sk, causal, wide):
     assert (form(b, h, hk, sq, sk, causal) == "wide") == wide
