@@ -759,7 +759,9 @@ hipError_t chunk_launch(const FmhaChunkArgs& a, int batch, int causal, hipStream
 //    shapes (S256-S8192, 192-3,072 blocks, us, other / wide): k = 2 B4 H16 S2048
 //    71 / 65, B64 H8 S256 17.2 / 15.5; k = 3 full B6 H16 S2048 108 / 98, B12 H16
 //    S1000 58 / 52; partial last rounds lose: B3 H16 S2048 (1.5 rounds) 56 / 60,
-//    B9 H16 S900 43.6 / 44.9, B8 H16 S1030 (an odd M-tile) 47.1 / 48.5.
+//    B9 H16 S900 43.6 / 44.9, B8 H16 S1030 (an odd M-tile) 47.1 / 48.5; causal, the
+//    regular form's at its mean M-tile: B28 H8/1 703 x 4872 220 / 208, B58 H8/2 S193
+//    (M-tiles of two and four tiles) 14.9 / 15.2.
 //    k = 1 is one wave per SIMD against the regular form's two: 3-6 % slower over
 //    490 shapes (H40 1024 x 512 11.7 / 12.4, H32 2048 x 256 8.6 / 9.6; a mask
 //    7-39 %), but where a head's two M-tiles fall on different XCDs (heads go
@@ -787,7 +789,9 @@ bool takes_wide(const FmhaFwdParams* p, int batch, int causal, int form, const D
         const int64_t k = (blocks + cus - 1) / cus;  // blocks of the fullest CU
         return two * (double)(k / 2) + one * (double)(k % 2);
     };
-    double other = us(regular, 1.12, 0.60);
+    // the regular form's M-tiles walk their own tiles, a wide block its last row's
+    const double mean = 0.5 * (mtile_tiles(p, causal, 0) + longest);
+    double other = us(regular, 1.12, 0.60) * (mean / longest);
     if (form == FMHA_VARIANT_PAIR) other = std::min(other, 1.065 * (double)(wide / cus));
     return us(wide, 1.86, 1.08) < 0.97 * other;
 }

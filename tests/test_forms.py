@@ -95,6 +95,8 @@ def test_workspace_and_form_agree():
 
 @pytest.mark.parametrize("b,h,hk,sq,sk,causal,wide", [
     (64, 8, 8, 256, 256, 0, True), (4, 16, 16, 2048, 2048, 0, True), (12, 16, 16, 1000, 1000, 0, True),  # two or more
+    (28, 8, 1, 703, 4872, 1, True), (12, 32, 32, 406, 1584, 1, True), (13, 8, 2, 1011, 4696, 1, True),
+    (58, 8, 2, 193, 193, 1, False), (50, 8, 2, 206, 206, 1, False), (26, 16, 4, 129, 129, 1, False),  # a light M-tile
     # at most one 256-row block per compute unit: one wave per SIMD
     (1, 40, 40, 1024, 512, 0, False), (1, 32, 32, 2048, 256, 0, False), (1, 64, 64, 767, 512, 0, False),
     (3, 24, 24, 445, 870, 1, False), (2, 16, 4, 1918, 1918, 0, False), (20, 4, 1, 389, 479, 1, False),
