@@ -372,7 +372,6 @@ __device__ __forceinline__ void decode_merge(const FmhaDecodeArgs& a) {
     for (int d = 1; d < 64; d <<= 1) lt += __shfl_xor(lt, d);
     const int sub = lane >> 4, col = 4 * (lane & 15);
     float4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 4
     for (int c0 = 0; c0 < n; c0 += 4) {  // loads past the last chunk repeat it, unused
         const int c = c0 + sub;
         const float wc = __shfl(w, c & 63);

@@ -742,9 +742,9 @@ hipError_t chunk_launch(const FmhaChunkArgs& a, int batch, int causal, hipStream
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (causal)
-        hipLaunchKernelGGL(fmha_fwd_d64_bf16_chunk_balanced_merge_msk1, merge, block, 0, stream, a);
+        hipLaunchKernelGGL(fmha_fwd_d64_bf16_chunk_merge_msk1, merge, block, 0, stream, a);
     else
-        hipLaunchKernelGGL(fmha_fwd_d64_bf16_chunk_balanced_merge_msk0, merge, block, 0, stream, a);
+        hipLaunchKernelGGL(fmha_fwd_d64_bf16_chunk_merge_msk0, merge, block, 0, stream, a);
     return hipGetLastError();
 }
 

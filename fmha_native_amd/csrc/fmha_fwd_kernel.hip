@@ -2340,10 +2340,10 @@ __device__ __forceinline__ void chunk_merge(const FmhaChunkArgs& a) {
         p.lse[((int64_t)b * p.nhead_q + h) * sq + row] =
             (__builtin_log2f(l) + m) * 0.69314718055994530942f;  // -inf when l == 0
 }
-__global__ __launch_bounds__(FMHA_KBLOCK) void fmha_fwd_d64_bf16_chunk_balanced_merge_msk0(FmhaChunkArgs args) {
+__global__ __launch_bounds__(FMHA_KBLOCK) void fmha_fwd_d64_bf16_chunk_merge_msk0(FmhaChunkArgs args) {
     chunk_merge<false>(args);
 }
-__global__ __launch_bounds__(FMHA_KBLOCK) void fmha_fwd_d64_bf16_chunk_balanced_merge_msk1(FmhaChunkArgs args) {
+__global__ __launch_bounds__(FMHA_KBLOCK) void fmha_fwd_d64_bf16_chunk_merge_msk1(FmhaChunkArgs args) {
     chunk_merge<true>(args);
 }
 

@@ -42,8 +42,8 @@ struct FmhaChunkArgs {
 };
 __global__ void fmha_fwd_d64_bf16_chunk_msk0(FmhaChunkArgs args);
 __global__ void fmha_fwd_d64_bf16_chunk_msk1(FmhaChunkArgs args);
-__global__ void fmha_fwd_d64_bf16_chunk_balanced_merge_msk0(FmhaChunkArgs args);
-__global__ void fmha_fwd_d64_bf16_chunk_balanced_merge_msk1(FmhaChunkArgs args);
+__global__ void fmha_fwd_d64_bf16_chunk_merge_msk0(FmhaChunkArgs args);
+__global__ void fmha_fwd_d64_bf16_chunk_merge_msk1(FmhaChunkArgs args);
 
 // Pair stream form (see fmha_fwd_kernel.hip): one 8-wave pair block per
 // compute unit looping over a static list of M-tile pairs.

@@ -22,15 +22,37 @@ _ENTRIES = [f"fmha_fwd_d64_bf16_{form}msk{m}{v}" for form in ("", "splitkv_", "p
             for m in (0, 1) for v in ("", "_varlen")]
 
 
-@pytest.fixture(scope="module")
-def asm(tmp_path_factory):
+# merges of partial results: no ring, every wave on its own rows
+_MERGES = ["fmha_fwd_d64_bf16_balanced_merge"] + [f"fmha_fwd_d64_bf16_chunk_merge_msk{m}" for m in (0, 1)] + \
+    [f"fmha_fwd_d64_bf16_decode_merge_msk{m}{v}" for m in (0, 1) for v in ("", "_varlen")]
+
+
+def _symbol(entry, args):
+    return f"_Z{len(entry)}{entry}{len(args)}{args}"
+
+
+_MERGE_SYMBOLS = {_symbol(e, "FmhaBalancedArgs" if "balanced" in e else "FmhaChunkArgs" if "chunk" in e
+                          else "FmhaDecodeArgs") for e in _MERGES}
+
+
+def _compile(tmp_path_factory, source):
     if shutil.which(build.HIPCC) is None and not os.path.exists(build.HIPCC):
         pytest.skip("hipcc not available")
     out = tmp_path_factory.mktemp("asm") / "kernel.s"
     cmd = [build.HIPCC, *[f for f in build.HIP_FLAGS if f != "-fPIC"], "--cuda-device-only", "-S",
-           os.path.join(build.CSRC, "fmha_fwd_kernel.hip"), "-o", str(out)]
+           os.path.join(build.CSRC, source), "-o", str(out)]
     subprocess.run(cmd, check=True, capture_output=True, text=True)
     return out.read_text()
+
+
+@pytest.fixture(scope="module")
+def asm(tmp_path_factory):
+    return _compile(tmp_path_factory, "fmha_fwd_kernel.hip")
+
+
+@pytest.fixture(scope="module")
+def decode_asm(tmp_path_factory):
+    return _compile(tmp_path_factory, "fmha_decode.hip")
 
 
 def _functions(src):
@@ -51,15 +73,17 @@ def test_every_entry_compiled(asm):
     for e in ("fmha_fwd_d64_bf16_balanced_msk1", "fmha_fwd_d64_bf16_balanced_pair_msk1",
               "fmha_fwd_d64_bf16_balanced_merge", "fmha_fwd_d64_bf16_pair_stream_msk0",
               "fmha_fwd_d64_bf16_pair_stream_msk1", "fmha_fwd_d64_bf16_msk1_varlen_tilemajor",
-              "fmha_fwd_d64_bf16_msk1_varlen_seqmajor"):
+              "fmha_fwd_d64_bf16_msk1_varlen_seqmajor", "fmha_fwd_d64_bf16_wide_msk013", "fmha_fwd_d64_bf16_wide_msk113",
+              "fmha_fwd_d64_bf16_wide_msk1_tilemajor", "fmha_fwd_d64_bf16_chunk_msk0", "fmha_fwd_d64_bf16_chunk_msk1",
+              "fmha_fwd_d64_bf16_chunk_merge_msk0", "fmha_fwd_d64_bf16_chunk_merge_msk1"):
         assert any(e in n for n in names), e
     for m in (0, 1):
         for v in ("", "_varlen"):
             assert any(f"fmha_fwd_d64_bf16_short_msk{m}{v}13FmhaFwdParams" in n for n in names), (m, v)
 
 
-def test_no_lds_read_in_flight_at_barriers(asm):
-    for name, body in _functions(asm).items():
+def test_no_lds_read_in_flight_at_barriers(asm, decode_asm):
+    for name, body in [*_functions(asm).items(), *_functions(decode_asm).items()]:
         pending, barriers = False, 0
         for line in body.splitlines():
             ins = line.strip()
@@ -70,16 +94,17 @@ def test_no_lds_read_in_flight_at_barriers(asm):
             elif ins.startswith("s_barrier"):
                 barriers += 1
                 assert not pending, f"{name}: LDS read in flight at barrier {barriers}"
-        # every attention entry synchronises its K/V ring; the balanced form's
-        # merge kernel has no ring (each wave stages its own rows)
-        assert barriers > 0 or "balanced_merge" in name, name
+        # every attention entry synchronises its K/V ring (decode: the waves'
+        # exchange of partial results)
+        assert (barriers == 0) == (name in _MERGE_SYMBOLS), name
 
 
-def test_no_scratch_and_two_waves_per_simd(asm):
-    scratch = re.findall(r"; ScratchSize: (\d+)", asm)
-    occupancy = re.findall(r"; Occupancy: (\d+)", asm)
-    assert scratch and all(int(s) == 0 for s in scratch), scratch
-    assert occupancy and all(int(o) >= 2 for o in occupancy), occupancy
+def test_no_scratch_and_two_waves_per_simd(asm, decode_asm):
+    for listing in (asm, decode_asm):
+        scratch = re.findall(r"; ScratchSize: (\d+)", listing)
+        occupancy = re.findall(r"; Occupancy: (\d+)", listing)
+        assert scratch and all(int(s) == 0 for s in scratch), scratch
+        assert occupancy and all(int(o) >= 2 for o in occupancy), occupancy
 
 
 def _occupancy(src):
@@ -165,3 +190,26 @@ def test_rowless_path_lies_behind_the_others(asm):
         bars = [i for i, x in enumerate(ins) if x.startswith("s_barrier")]
         assert any(x.startswith("v_mfma") for x in ins[bars[0]:bars[1]]), name
     assert seen == 7  # regular, split-KV and pair, each also varlen; chunk
+
+
+def test_decode_entries(decode_asm):
+    """Eight walk entries (eight or four waves: 128 or 64 KiB of LDS, so one or
+    two blocks and two waves per SIMD) and four merges.  Every step of a walk's
+    loop issues the next step's eight loads, and the wait between them and the
+    step's LDS reads leaves those eight in flight."""
+    funcs, occ, lds = _functions(decode_asm), _occupancy(decode_asm), _lds_bytes(decode_asm)
+    walks = {n: b for n, b in funcs.items() if n not in _MERGE_SYMBOLS}
+    assert set(funcs) - set(walks) == {n for n in _MERGE_SYMBOLS if "decode" in n} and len(walks) == 8
+    for name, body in walks.items():
+        assert occ[name] == 2 and lds[name] == (64 if "decode4" in name else 128) * 1024, name
+        ins = [ln.strip() for ln in body.splitlines() if ln.strip() and not ln.strip().startswith((";", "."))]
+        is_dma = [x.startswith("buffer_load_dwordx4") and x.endswith(" lds") for x in ins]
+        first = next(i for i, x in enumerate(ins) if x.startswith("ds_read"))
+        last = max(i for i, x in enumerate(ins) if x.startswith("v_mfma"))
+        waits, since = [], 0
+        for i in range(first + 1, last):  # the loop, and what the compiler laid out between its parts
+            since = since + 1 if is_dma[i] else since
+            if "vmcnt" in ins[i] and ins[i].startswith("s_waitcnt"):
+                waits.append((int(re.search(r"vmcnt\((\d+)\)", ins[i]).group(1)), since))
+                since = 0
+        assert waits == [(8, 8), (8, 8)], (name, waits)  # the two ring stages' steps

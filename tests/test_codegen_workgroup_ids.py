@@ -30,7 +30,7 @@ import pytest
 
 from fmha_native_amd import build
 
-_SOURCES = ["fmha_fwd_kernel.hip", "fmha_merge.hip"]
+_SOURCES = ["fmha_fwd_kernel.hip", "fmha_decode.hip", "fmha_merge.hip"]
 
 
 def _device_asm(tmp_path, name):
