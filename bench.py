@@ -387,8 +387,8 @@ def _roofline(achieved, workload, ms_per_step):
     HBM traffic, MFMA busy and the clock from the committed rocprofv3 run of
     the same kernel (one box, one process tree), where
     frac_from_counters = mfma_busy x clock / 2.4 GHz checks the timer.  The
-    kernel is cycle-bound (the same active cycles per launch on every box
-    measured), so those cycles over a run's time per launch give the clock
+    kernel is cycle-bound (the same active cycles per launch within 0.3 % on
+    every box a form was counted on), so those cycles over a run's time per launch give the clock
     that box held: this run's frac over the profile run's is the ratio of the
     two clocks."""
     prof = _profile(workload)
