@@ -762,9 +762,9 @@ hipError_t chunk_launch(const FmhaChunkArgs& a, int batch, int causal, hipStream
 //    B9 H16 S900 43.6 / 44.9, B8 H16 S1030 (an odd M-tile) 47.1 / 48.5; causal, the
 //    regular form's at its mean M-tile: B28 H8/1 703 x 4872 220 / 208, B58 H8/2 S193
 //    (M-tiles of two and four tiles) 14.9 / 15.2.
-//    k = 1 is one wave per SIMD against the regular form's two: 3-6 % slower over
-//    490 shapes (H40 1024 x 512 11.7 / 12.4, H32 2048 x 256 8.6 / 9.6; a mask
-//    7-39 %), but where a head's two M-tiles fall on different XCDs (heads go
+//    k = 1 is one wave per SIMD against the regular form's two: 2-5 % slower at the
+//    quartiles of 260 unmasked shapes, 2-29 % of 50 masked ones (H40 1024 x 512
+//    11.7 / 12.4, H32 2048 x 256 8.6 / 9.6), but where a head's two M-tiles fall on different XCDs (heads go
 //    round robin) and its keys are few, one block reads them once: B26 H6 153 x
 //    848 20.0 / 17.6, B54 H4/1 132 x 1159 27.1 / 24.3, B14 H12 238 x 238 10.5 /
 //    9.4; past 20 key tiles 0.86-1.10x, up to two 0.84-1.07x (H129 256 x 64 5.7 /

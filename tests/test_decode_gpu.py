@@ -1,5 +1,6 @@
 """Decode form: packed query rows of a KV head over many keys, whole or split
 over key chunks, against float64 attention."""
+import ctypes
 import math
 
 import numpy as np
@@ -251,3 +252,29 @@ def test_workspace_outlives_the_call_on_another_stream(monkeypatch):
     assert again.data_ptr() + need <= ptr or ptr + need <= again.data_ptr()
     torch.cuda.synchronize()
     del out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("h,hk,sq,sk", [(8, 8, 3, 9001), (4, 4, 700, 700), (4, 4, 4161, 4161), (2, 2, 9000, 9000)])
+def test_static_array_gives_the_plans_bytes_or_none(h, hk, sq, sk):
+    """The entry point on the static array runs what a workspace of the
+    balanced plan's bytes (0 without a plan) runs, bit for bit: decode, split
+    and whole, chunk and balanced."""
+    g = torch.Generator(device="cuda").manual_seed(sk)
+    rnd = lambda n, s: torch.randn((1, n, s, 64), generator=g, device="cuda").to(torch.bfloat16)
+    q, k, v = rnd(h, sq), rnd(hk, sk), rnd(hk, sk)
+    lib, stream = fmha.load_library(), torch.cuda.current_stream().cuda_stream
+    outs = []
+    for entry in ("ws", "noalloc"):
+        o, lse = torch.full_like(q, float("nan")), torch.full(q.shape[:-1], float("nan"), device="cuda")
+        p = fmha.params_from_tensors(q, k, v, o, lse)
+        plan = fmha.workspace_size(p, 1, 1, fmha.VARIANT_REFERENCE_ORDER)  # the flag leaves the balanced form alone
+        ws = torch.empty(max(plan, 256), dtype=torch.uint8, device="cuda")
+        if entry == "ws":
+            fmha.fmha_fwd_d64_bf16_ws(p, 1, 1, ws.data_ptr() if plan else None, plan, stream)
+        else:
+            assert lib.fmha_fwd_d64_bf16_noalloc(ctypes.byref(p), 1, 1, fmha.VARIANT_AUTO, stream) == 0
+        torch.cuda.synchronize()
+        outs.append((o, lse))
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+    _check(outs[1][0][0], outs[1][1][0], *_f64(q[0], k[0], v[0], 1), (sq, sk))
